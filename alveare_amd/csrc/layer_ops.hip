@@ -21,9 +21,9 @@
 // Attention is not bit-exact: the reference's scores and weighted sums are
 // BLAS dot products (np.dot) whose order is the library's. Here the positions
 // are split into chunks of 64: a workgroup per (chunk, kv head, group of up
-// to 4 q heads) writes the chunk's max, exp-sum and weighted V sum to the
-// stream's scratch, and a second launch merges the chunks of every (head,
-// column) in chunk order (deterministic).
+// to 4 q heads; 16 for long spans of 512-wide heads) writes the chunk's max,
+// exp-sum and weighted V sum to the stream's scratch, and a second launch
+// merges the chunks of every (head, column) in chunk order (deterministic).
 //
 // Row kernels run 256 threads per row: 16-byte loads and stores, and the
 // pairwise sum with 8 lanes per leaf (lane j holds the leaf's accumulator
@@ -258,7 +258,7 @@ struct AttnArgs {
     const uint16_t* kcache;
     const uint16_t* vcache;
     uint16_t* out;      // [heads][D]
-    int heads, kv_heads, D, max_seq, window, hg;
+    int heads, kv_heads, D, max_seq, window, g;  // g: q heads per kv head
     float scale;
     const int* pos;
     int nchunk;          // grid.x: chunks the largest window can need
@@ -307,7 +307,7 @@ __global__ void __launch_bounds__(kAttnThreads) attn_partial_kernel(AttnArgs a) 
     __shared__ __align__(16) float red[PG * HG * D];  // [pg][head][D]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = blockIdx.x, kvh = blockIdx.y;
-    const int g = a.heads / a.kv_heads;
+    const int g = a.g;
     const int h0 = blockIdx.z * HG;
     const int pos = *a.pos;
     if (pos < 0 || pos >= a.max_seq) return;
@@ -538,42 +538,393 @@ __global__ void __launch_bounds__(kAttnThreads) attn_partial_kernel(AttnArgs a) 
     }
 }
 
-// Head blockIdx.x, columns [256 blockIdx.y, + 256): the chunks merged in order,
-// out = sum_c o_c f_c / sum_c l_c f_c with f_c = exp(m_c - max_c m_c).
-__global__ void __launch_bounds__(kAttnThreads) attn_merge_kernel(AttnArgs a) {
+// Sixteen q heads per workgroup at D = 512, for long spans, on the matrix
+// cores: K and V read once instead of once per two heads, and every result bit
+// that of the partial kernel. v_mfma_f32_16x16x4_f32 adds its four products in
+// order, each by one fused multiply-add (checked against fmaf on random data
+// down to subnormals, test_attention_wide_bit_identical), so a chain of them
+// over k is the chain of fmaf it replaces. A = the 16 heads' q values (weights),
+// B = 16 positions' K values (16 columns' V values), widened from bf16.
+//   * Scores: wave w takes quarter w % 4 of the columns (the partial kernel's
+//     four chains per score) for two of the four 16-position tiles.
+//   * V sum: wave w takes 64 columns; its four accumulators per column are the
+//     partial kernel's position groups, then added in order.
+//   * Lane group gq of a step holds k = 4 s + gq: K rows and q rows sit in LDS
+//     with the pair (k, k + 4) of each octet in one dword and the pairs of one
+//     gq together (four byte permutes per octet), so a 16-byte read feeds eight
+//     steps. V goes straight to registers.
+// 16 q heads on one kv head, 12002 positions: 17.7 us against 65 for the two-head
+// workgroups (197 MB of rows through the L2s); 188 workgroups, whose rows' 25 MB
+// take 4 of them, the rest is the chain of one chunk's steps: position 1, loads
+// and norms 4, scores 2.5, softmax 1, V sum 2.5, stores 0.5.
+constexpr int kWideHeads = 16;
+constexpr int kWideD = 512;
+constexpr int kWideThreads = 512;
+constexpr long kWideMinGrid = 64;
+constexpr int kWideRow = 2 * kWideD + 16;  // LDS bytes of a K or q row: 16 rows' pieces in different banks
+constexpr int kWideScore = kAttnChunk + 4; // floats of a score row, likewise
+// Dynamic LDS: K rows, q rows, the new v row, max and exp-sum, then the score
+// quarters (later the weights), in whose place the post-processing keeps two
+// float rows per wave.
+constexpr int kWideScoreFloats = 4 * kWideHeads * kWideScore;
+constexpr int kWideRowFloats = 2 * (kWideThreads / 64) * kWideD;
+constexpr int kWideLds = kAttnChunk * kWideRow + kWideHeads * kWideRow + 2 * kWideD + 2 * kWideHeads * 4 +
+                         4 * (kWideScoreFloats > kWideRowFloats ? kWideScoreFloats : kWideRowFloats);
+
+// Octet p of a row into its LDS row (bytes): dword gq * 64 + p = values gq, gq + 4.
+__device__ __forceinline__ void put_octet(unsigned char* row, int p, uint4 v) {
+    uint32_t* d = reinterpret_cast<uint32_t*>(row) + p;
+    d[0] = __builtin_amdgcn_perm(v.z, v.x, 0x05040100u);
+    d[64] = __builtin_amdgcn_perm(v.z, v.x, 0x07060302u);
+    d[128] = __builtin_amdgcn_perm(v.w, v.y, 0x05040100u);
+    d[192] = __builtin_amdgcn_perm(v.w, v.y, 0x07060302u);
+}
+__device__ __forceinline__ float lo_bf16(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
+__device__ __forceinline__ float hi_bf16(uint32_t w) { return __builtin_bit_cast(float, w & 0xFFFF0000u); }
+
+template <bool FQ>
+__global__ void __launch_bounds__(kWideThreads) attn_wide_kernel(AttnArgs a) {
+    constexpr int D = kWideD, HG = kWideHeads, NWV = kWideThreads / 64;
+    constexpr int RW = D / 64;  // row elements per lane, lane l: [RW l, RW l + RW)
+    constexpr int NK = kAttnChunk / NWV;
+    static_assert(RW == 8 && 256 / (D / 8) == 4, "an octet per lane, four position groups");
+    extern __shared__ __align__(16) unsigned char wsm[];
+    unsigned char* ktile = wsm;
+    unsigned char* qs = ktile + kAttnChunk * kWideRow;
+    uint16_t* vn = reinterpret_cast<uint16_t*>(qs + HG * kWideRow);
+    float* mls = reinterpret_cast<float*>(vn + D);
+    float* sc = mls + 2 * HG;  // [quarter][head][position]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15, gq = lane >> 4;
+    const int c = blockIdx.x, kvh = blockIdx.y;
+    const int g = a.g;
+    const int h0 = blockIdx.z * HG;
+    const int pos = *a.pos;
+    if (pos < 0 || pos >= a.max_seq) return;
+    const AttnSpan sp = attn_span(a, pos);
+    if (c >= sp.nch) return;
+    const int p0 = c * kAttnChunk;
+    const int np = min(kAttnChunk, sp.W - p0);
+    const size_t row0 = (size_t)kvh * a.max_seq + sp.start + p0;
+    const bool lastc = c == sp.nch - 1;
+    const int nold = FQ && lastc ? np - 1 : kAttnChunk;  // rows from here on are the new k and v, not the caches'
+
+    // Rows of the post-processing: wave + 8 t, the q heads then (in the chunk
+    // that holds pos) k and v, all loaded before K and V.
+    uint16_t xraw[3][RW], craw[RW], sraw[RW];
+    float wraw[2][RW];
+    const bool kvrow = FQ && lastc && wave < 2;  // k (wave 0), v (wave 1)
+    if constexpr (FQ) {
+        const QkvPostArgs& pa = a.post;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+            __builtin_memcpy(xraw[t], pa.qkv + (kvh * g + h0 + wave + NWV * t) * D + RW * lane, sizeof(xraw[t]));
+        if (pa.q_w) __builtin_memcpy(wraw[0], pa.q_w + RW * lane, sizeof(wraw[0]));
+        if (kvrow) {
+            __builtin_memcpy(xraw[2], pa.qkv + (wave == 0 || pa.v_off < 0 ? pa.k_off : pa.v_off) + kvh * D + RW * lane,
+                             sizeof(xraw[2]));
+            if (pa.k_w) __builtin_memcpy(wraw[1], pa.k_w + RW * lane, sizeof(wraw[1]));
+        }
+        if (pa.rope) {
+            const uint16_t* rr = pa.rope + (size_t)pos * pa.rope_stride;
+            if (pa.half % RW == 0) {
+                const int i = (RW * lane) % pa.half;
+                __builtin_memcpy(craw, rr + pa.cos_off + i, sizeof(craw));
+                __builtin_memcpy(sraw, rr + pa.sin_off + i, sizeof(sraw));
+            } else {
+#pragma unroll
+                for (int e = 0; e < RW; ++e) {
+                    const int i = (RW * lane + e) % pa.half;
+                    craw[e] = rr[pa.cos_off + i];
+                    sraw[e] = rr[pa.sin_off + i];
+                }
+            }
+        }
+        asm volatile("" ::: "memory");  // these loads go out before the K and V loads
+    }
+    // K: octet `lane` of rows wave + 8 i. V: columns vcol .. + 3 of positions
+    // 16 s + 4 gq + pg. Rows past the chunk's end read its last row.
+    const int vcol = 64 * wave + 4 * j;
+    uint4 kreg[NK];
+    uint2 vreg[4][4];  // [s][pg]
+    {
+        const uint4* kr = reinterpret_cast<const uint4*>(a.kcache + row0 * D) + lane;
+#pragma unroll
+        for (int i = 0; i < NK; ++i) kreg[i] = kr[(uint32_t)(min(wave + NWV * i, np - 1) * (D / 8))];
+        asm volatile("" ::: "memory");
+        const uint2* vr = reinterpret_cast<const uint2*>(a.vcache + row0 * D + vcol);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int pg = 0; pg < 4; ++pg) vreg[s][pg] = vr[(uint32_t)(min(16 * s + 4 * gq + pg, np - 1) * (D / 4))];
+        asm volatile("" ::: "memory");
+    }
+    if constexpr (FQ) {
+        // NR rows side by side (a row is one chain of dependent steps, two
+        // take what one does): its values v, norm weights w, role 0 a q head,
+        // 1 k, 2 v.
+        const QkvPostArgs& pa = a.post;
+        auto do_rows = [&](auto nr, int role, const uint16_t (*x)[RW], const float (&w)[RW]) __attribute__((always_inline)) {
+            constexpr int NR = decltype(nr)::value;
+            const int norm = role == 0 ? pa.norm_q : (role == 1 ? pa.norm_k : pa.norm_v);
+            const bool hasw = role == 0 ? pa.q_w != nullptr : (role == 1 ? pa.k_w != nullptr : false);
+            float v[NR][RW];
+            auto row = [&](int t) __attribute__((always_inline)) { return sc + (2 * wave + t) * D; };
+            auto put = [&](int t) __attribute__((always_inline)) {
+                float4* p = reinterpret_cast<float4*>(row(t)) + 2 * lane;
+                p[0] = float4{v[t][0], v[t][1], v[t][2], v[t][3]};
+                p[1] = float4{v[t][4], v[t][5], v[t][6], v[t][7]};
+            };
+#pragma unroll
+            for (int t = 0; t < NR; ++t) {
+#pragma unroll
+                for (int e = 0; e < RW; ++e) v[t][e] = bf16_bits_to_f32(x[t][e]);
+                put(t);
+            }
+            if (norm) {
+                float inv[NR];
+#pragma unroll
+                for (int t = 0; t < NR; ++t) inv[t] = rms_inv_wave(row(t), D, pa.eps, lane);
+#pragma unroll
+                for (int t = 0; t < NR; ++t) {
+#pragma unroll
+                    for (int e = 0; e < RW; ++e) {
+                        const float tt = mul_rn(v[t][e], inv[t]);
+                        v[t][e] = bf16r(hasw ? mul_rn(tt, w[e]) : tt);
+                    }
+                    put(t);
+                }
+            }
+            const bool rot = role < 2 && pa.rope;
+            const int d0 = RW * lane;
+#pragma unroll
+            for (int t = 0; t < NR; ++t) {
+                float other[RW];  // the other value of each rotated pair
+                if (rot) {
+                    if (pa.half % RW == 0) {
+                        const float4* op = reinterpret_cast<const float4*>(
+                            row(t) + (d0 < pa.half ? d0 + pa.half : d0 < 2 * pa.half ? d0 - pa.half : d0));
+                        const float4 o0 = op[0], o1 = op[1];
+                        const float t8[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
+                        __builtin_memcpy(other, t8, sizeof(other));
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < RW; ++e) {
+                            const int d = d0 + e;
+                            other[e] = row(t)[d < pa.half ? d + pa.half : d < 2 * pa.half ? d - pa.half : d];
+                        }
+                    }
+                }
+                uint16_t ob[RW];
+#pragma unroll
+                for (int e = 0; e < RW; ++e) {
+                    const int d = d0 + e;
+                    float y = v[t][e];
+                    if (rot) {
+                        // run_rope_cpu_gemma (model.py:549-575): y1 = x1 c - x2 s, y2 = x2 c + x1 s.
+                        const float cr = mul_rn(y, bf16_bits_to_f32(craw[e])), sr = mul_rn(other[e], bf16_bits_to_f32(sraw[e]));
+                        const float z = d < pa.half ? sub_rn(cr, sr) : add_rn(cr, sr);
+                        y = d < 2 * pa.half ? z : y;
+                    }
+                    ob[e] = bf16_rne_bits(y);
+                }
+                const uint4 o8 = pack8(ob);
+                if (role == 0) {
+                    const int r = wave + NWV * t;
+                    put_octet(qs + r * kWideRow, lane, o8);
+                    if (c == 0 && pa.q_out)
+                        __builtin_memcpy(pa.q_out + (size_t)(kvh * g + h0 + r) * D + d0, &o8, sizeof(o8));
+                } else {
+                    if (role == 1)
+                        put_octet(ktile + (np - 1) * kWideRow, lane, o8);
+                    else
+                        reinterpret_cast<uint4*>(vn)[lane] = o8;
+                    if (blockIdx.z == 0)
+                        __builtin_memcpy((role == 1 ? pa.kcache : pa.vcache) + ((size_t)kvh * a.max_seq + pos) * D + d0, &o8,
+                                         sizeof(o8));
+                }
+            }
+        };
+        do_rows(std::integral_constant<int, 2>{}, 0, xraw, wraw[0]);
+        if (kvrow) do_rows(std::integral_constant<int, 1>{}, 1 + wave, xraw + 2, wraw[1]);
+    } else {
+        const uint4* qv = reinterpret_cast<const uint4*>(a.q + ((size_t)kvh * g + h0) * D) + lane;
+#pragma unroll
+        for (int t = 0; t < HG / NWV; ++t) put_octet(qs + (wave + NWV * t) * kWideRow, lane, qv[(wave + NWV * t) * (D / 8)]);
+    }
+#pragma unroll
+    for (int i = 0; i < NK; ++i)
+        if (wave + NWV * i < nold) put_octet(ktile + (wave + NWV * i) * kWideRow, lane, kreg[i]);
+    __syncthreads();
+
+    // Scores of positions 32 (wave / 4) + 16 u + j, quarter wave % 4 of the
+    // columns. (Rows past the chunk's end hold anything; their scores are not read.)
+    {
+        const int quarter = wave & 3, t0 = 2 * (wave >> 2);
+        f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+        const uint4* qp = reinterpret_cast<const uint4*>(qs + j * kWideRow + 256 * gq + 64 * quarter);
+        const uint4* kp0 = reinterpret_cast<const uint4*>(ktile + (16 * t0 + j) * kWideRow + 256 * gq + 64 * quarter);
+        const uint4* kp1 = kp0 + 16 * kWideRow / 16;
+        auto steps = [&](uint32_t q, uint32_t k0, uint32_t k1) __attribute__((always_inline)) {
+            s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(lo_bf16(q), lo_bf16(k0), s[0], 0, 0, 0);
+            s[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(lo_bf16(q), lo_bf16(k1), s[1], 0, 0, 0);
+            s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(hi_bf16(q), hi_bf16(k0), s[0], 0, 0, 0);
+            s[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(hi_bf16(q), hi_bf16(k1), s[1], 0, 0, 0);
+        };
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const uint4 q = qp[m], k0 = kp0[m], k1 = kp1[m];
+            steps(q.x, k0.x, k1.x);
+            steps(q.y, k0.y, k1.y);
+            steps(q.z, k0.z, k1.z);
+            steps(q.w, k0.w, k1.w);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sc[(quarter * HG + 4 * gq + r) * kWideScore + 16 * (t0 + u) + j] = s[u][r];
+    }
+    __syncthreads();
+
+    // The chunk's softmax pieces: two heads per wave; positions past the
+    // chunk's end weigh zero.
+#pragma unroll
+    for (int t = 0; t < HG / NWV; ++t) {
+        const int h = wave + NWV * t;
+        auto quarter = [&](int q) { return sc[(q * HG + h) * kWideScore + lane]; };
+        const float v = (quarter(0) + quarter(1)) + (quarter(2) + quarter(3));
+        const float s = lane < np ? v * a.scale : -__builtin_inff();
+        float m = s;
+        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+        const float e = lane < np ? expf(s - m) : 0.0f;
+        float l = e;
+        for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
+        sc[h * kWideScore + lane] = e;
+        if (lane == 0) {
+            mls[2 * h] = m;
+            mls[2 * h + 1] = l;
+        }
+    }
+    __syncthreads();
+
+    // Weighted V sum: position group pg holds positions pg, pg + 4, ... (those
+    // past the chunk's end weigh zero).
+    constexpr int gstride = D + 2;
+    float* out = a.part + (((size_t)kvh * a.nchunk + c) * g + h0) * gstride;
+    {
+        f32x4 o[4][4];  // [column vcol + e][pg]
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int pg = 0; pg < 4; ++pg) o[e][pg] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const float4 wv = *reinterpret_cast<const float4*>(sc + j * kWideScore + 16 * s + 4 * gq);
+            const float w[4] = {wv.x, wv.y, wv.z, wv.w};
+#pragma unroll
+            for (int pg = 0; pg < 4; ++pg) {
+                uint2 v = vreg[s][pg];
+                if (16 * s + 4 * gq + pg >= nold) v = *reinterpret_cast<const uint2*>(vn + vcol);
+                o[0][pg] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[pg], lo_bf16(v.x), o[0][pg], 0, 0, 0);
+                o[1][pg] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[pg], hi_bf16(v.x), o[1][pg], 0, 0, 0);
+                o[2][pg] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[pg], lo_bf16(v.y), o[2][pg], 0, 0, 0);
+                o[3][pg] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[pg], hi_bf16(v.y), o[3][pg], 0, 0, 0);
+            }
+        }
+        // Lane (j, gq) holds heads 4 gq + r.
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float y[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                y[e] = 0.0f;
+#pragma unroll
+                for (int pg = 0; pg < 4; ++pg) y[e] += o[e][pg][r];
+            }
+            float2* dst = reinterpret_cast<float2*>(out + (size_t)(4 * gq + r) * gstride + vcol);
+            dst[0] = float2{y[0], y[1]};
+            dst[1] = float2{y[2], y[3]};
+        }
+    }
+    if (tid < HG) *reinterpret_cast<float2*>(out + (size_t)tid * gstride + D) = float2{mls[2 * tid], mls[2 * tid + 1]};
+}
+
+// Head blockIdx.x, columns [64 blockIdx.y, + 64): the chunks merged in order,
+// out = sum_c o_c f_c / sum_c l_c f_c with f_c = exp(m_c - max_c m_c). The
+// factors are evaluated by all threads and the chunks' values staged in LDS
+// by all of them, kMergeStage chunks at a time (48 KiB); one thread per column
+// (and one for the denominator) then adds in chunk order. 188 chunks of 16
+// heads of 512: 6 us; with one thread evaluating the factors and 32 workgroups
+// of 256 columns, 8 loads in flight each, 20.
+constexpr int kMergeThreads = 512;
+constexpr int kMergeStage = 192;
+
+__global__ void __launch_bounds__(kMergeThreads) attn_merge_kernel(AttnArgs a) {
+    constexpr int NW = kMergeThreads / 64, NB = 8;  // NB: loads per batch
     __shared__ float fs[kAttnMaxChunks], lsum[kAttnMaxChunks];
-    __shared__ float Ls;
-    const int tid = threadIdx.x;
+    __shared__ float os[kMergeStage][64];
+    __shared__ float red[NW], Ls;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hq = blockIdx.x;
-    const int g = a.heads / a.kv_heads, kvh = hq / g, hl = hq - kvh * g;
+    const int g = a.g, kvh = hq / g, hl = hq - kvh * g;
     const int D = a.D, gstride = D + 2;
     const int pos = *a.pos;
     if (pos < 0 || pos >= a.max_seq) return;
     const int nch = attn_span(a, pos).nch;
     const float* base = a.part + ((size_t)kvh * a.nchunk * g + hl) * gstride;  // chunk q at + q * g * gstride
-    for (int q = tid; q < nch; q += kAttnThreads) {
+    const float* col = base + blockIdx.y * 64 + lane;
+    // Chunks [q0, q0 + kMergeStage) of the 64 columns, every load of a wave in
+    // flight at once (a chunk past the last reads it again).
+    auto stage = [&](int q0) __attribute__((always_inline)) {
+        const int n = min(nch - q0, kMergeStage);
+        float v[kMergeStage / NW];
+#pragma unroll
+        for (int b = 0; b < kMergeStage / NW; b += NB)
+            if (wave + NW * b < n)
+#pragma unroll
+                for (int t = b; t < b + NB; ++t) v[t] = col[(size_t)(q0 + min(wave + NW * t, n - 1)) * g * gstride];
+#pragma unroll
+        for (int b = 0; b < kMergeStage / NW; b += NB)
+            if (wave + NW * b < n)
+#pragma unroll
+                for (int t = b; t < b + NB; ++t) os[wave + NW * t][lane] = v[t];
+    };
+    float m = -__builtin_inff();
+    for (int q = tid; q < nch; q += kMergeThreads) {
         fs[q] = base[(size_t)q * g * gstride + D];
         lsum[q] = base[(size_t)q * g * gstride + D + 1];
+        m = fmaxf(m, fs[q]);
     }
+    stage(0);
+    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    if (lane == 0) red[wave] = m;
     __syncthreads();
-    if (tid == 0) {
-        float M = -__builtin_inff();
-        for (int q = 0; q < nch; ++q) M = fmaxf(M, fs[q]);
-        float L = 0.0f;
-        for (int q = 0; q < nch; ++q) {
-            const float f = expf(fs[q] - M);
-            L = fmaf(lsum[q], f, L);
-            fs[q] = f;
-        }
-        Ls = L;
-    }
+#pragma unroll
+    for (int w = 0; w < NW; ++w) m = fmaxf(m, red[w]);
+    for (int q = tid; q < nch; q += kMergeThreads) fs[q] = expf(fs[q] - m);
     __syncthreads();
-    const int d = blockIdx.y * kAttnThreads + tid;
-    if (d >= D) return;
     float O = 0.0f;
+    for (int q0 = 0; q0 < nch; q0 += kMergeStage) {
+        if (q0) {
+            __syncthreads();
+            stage(q0);
+            __syncthreads();
+        }
+        const int n = min(nch - q0, kMergeStage);
+        if (wave == 0) {
 #pragma unroll 8
-    for (int q = 0; q < nch; ++q) O = fmaf(base[(size_t)q * g * gstride + d], fs[q], O);
-    a.out[(size_t)hq * D + d] = bf16_rne_bits(__fdiv_rn(O, Ls));
+            for (int q = 0; q < n; ++q) O = fmaf(os[q][lane], fs[q0 + q], O);
+        } else if (wave == 1 && q0 == 0) {
+            float L = 0.0f;
+#pragma unroll 8
+            for (int q = 0; q < nch; ++q) L = fmaf(lsum[q], fs[q], L);
+            if (lane == 0) Ls = L;
+        }
+    }
+    __syncthreads();
+    if (wave == 0) a.out[(size_t)hq * D + blockIdx.y * 64 + lane] = bf16_rne_bits(__fdiv_rn(O, Ls));
 }
 
 // ---- alv_add_norm --------------------------------------------------------------
@@ -801,9 +1152,18 @@ int launch_attention(AttnArgs& a, bool fused, hipStream_t s) {
     const size_t part_bytes = (size_t)kv_heads * nchunk * g * (D + 2) * sizeof(float);
     void* sc = nullptr;
     if (int rc = get_scratch(s, kScratchAttn, part_bytes, &sc)) return rc;
-    a.hg = hg;
     a.nchunk = nchunk;
     a.part = static_cast<float*>(sc);
+    // Sixteen heads per workgroup (attn_wide_kernel) where the longest span
+    // leaves 64 workgroups or more (a 4096-position cache on one kv head).
+    // Both calls' launches, us, 16 heads on one kv head, two heads per
+    // workgroup against sixteen: 2048-position cache 14.8 against 16.4 at
+    // position 1500; 4096: 15.1 / 16.5 at 1500, 25.8 / 18.7 at 4000; 12288:
+    // 16.5 / 16.5 at 1500, 64.7 / 23.4 at 12000; 32768: 20.4 / 16.4 at 1500,
+    // 166 / 47 at 32000.
+    const bool wide = D == kWideD && g % kWideHeads == 0 && (long)nchunk * kv_heads * (g / kWideHeads) >= kWideMinGrid;
+    if (wide) hg = kWideHeads;
+    a.g = g;
     const dim3 grid(nchunk, kv_heads, g / hg);
     const void* k = nullptr;
     auto pick = [&](auto d, auto f) {
@@ -826,14 +1186,21 @@ int launch_attention(AttnArgs& a, bool fused, hipStream_t s) {
             default: pick(std::integral_constant<int, 512>{}, f); break;
         }
     };
-    if (fused)
+    int threads = kAttnThreads, lds = 0;
+    if (wide) {
+        k = fused ? reinterpret_cast<const void*>(&attn_wide_kernel<true>)
+                  : reinterpret_cast<const void*>(&attn_wide_kernel<false>);
+        threads = kWideThreads;
+        lds = kWideLds;
+        if (int rc = hip_check(set_lds(k, lds), "hipFuncSetAttribute")) return rc;
+    } else if (fused)
         pick_d(std::true_type{});
     else
         pick_d(std::false_type{});
     void* kargs[] = {&a};
-    if (int rc = hip_check(hipLaunchKernel(k, grid, dim3(kAttnThreads), kargs, 0, s), "attn_partial_kernel launch"))
+    if (int rc = hip_check(hipLaunchKernel(k, grid, dim3(threads), kargs, lds, s), "attn_partial_kernel launch"))
         return rc;
-    hipLaunchKernelGGL(attn_merge_kernel, dim3(heads, (D + kAttnThreads - 1) / kAttnThreads), dim3(kAttnThreads), 0, s, a);
+    hipLaunchKernelGGL(attn_merge_kernel, dim3(heads, D / 64), dim3(kMergeThreads), 0, s, a);
     return hip_check(hipGetLastError(), "attn_merge_kernel launch");
 }
 

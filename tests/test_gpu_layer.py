@@ -238,6 +238,47 @@ def test_qkv_attention_fused_bit_identical(dev, sliding, pos):
     assert np.array_equal(bf_np(vc_a), bf_np(vc_b))
 
 
+@pytest.mark.parametrize("pos,window,heads,half,v_off", [(0, 0, 16, 256, -1), (1, 0, 16, 64, 0), (62, 0, 32, 0, -1),
+                                                          (63, 0, 16, 256, 0), (64, 0, 16, 37, 0), (500, 100, 16, 256, 0),
+                                                          (2047, 0, 16, 256, -1), (2047, 0, 32, 256, 0)])
+def test_attention_wide_bit_identical(dev, pos, window, heads, half, v_off):
+    """From a 4096-position cache on, 16 q heads of 512 per workgroup on the
+    matrix cores give, bit for bit, what the two-head workgroups of a
+    2048-position cache give on the same rows: attention output, rotated q and
+    both cache rows, through both entry points (chunk edges, one position, a
+    window, two workgroups per chunk, RoPE of all, some and no values)."""
+    from alveare_amd import layer
+
+    _say(f"wide attention pos={pos} window={window} heads={heads} half={half}")
+    D, S, wide = 512, 2048, 4096
+    rng = np.random.default_rng(pos + heads + half)
+    qkv = bf_dev(rnd_bf16(rng, (heads + 2) * D, 1.0), dev)
+    kc0, vc0 = rnd_bf16(rng, (1, S, D), 0.2), rnd_bf16(rng, (1, S, D), 1.0)
+    qw, kw = rng.uniform(0.1, 0.3, D).astype(np.float32), rng.uniform(0.1, 0.3, D).astype(np.float32)
+    pos_dev = torch.tensor([pos], dtype=torch.int32, device=dev)
+    got = []
+    for rows in (S, wide):
+        kc = torch.zeros((1, rows, D), dtype=torch.bfloat16, device=dev)
+        vc = torch.zeros_like(kc)
+        kc[:, :S] = bf_dev(kc0, dev).view(1, S, D)
+        vc[:, :S] = bf_dev(vc0, dev).view(1, S, D)
+        kc[:, pos] = float("nan")  # the fused call must not use what the caches held there
+        vc[:, pos] = float("nan")
+        table = bf_dev(rnd_bf16(np.random.default_rng(7), (wide, 2 * 256), 1.0), dev).view(wide, 512)[:rows].contiguous()
+        rope = dict(rope=table, rope_stride=512, cos_off=0, sin_off=256, half=half) if half else {}
+        q = torch.empty(heads * D, dtype=torch.bfloat16, device=dev)
+        out = layer.qkv_attention(qkv, pos_dev, kc, vc, heads=heads, kv_heads=1, D=D, k_off=heads * D,
+                                  v_off=(heads + 1) * D if v_off >= 0 else -1, q_w=qw, k_w=kw, q_out=q, window=window,
+                                  **rope)
+        again = layer.attention(q, kc, vc, pos_dev, heads=heads, window=window)
+        torch.cuda.synchronize()
+        assert np.array_equal(bf_np(out), bf_np(again))
+        got.append([bf_np(t) for t in (out, q, kc[:, pos].contiguous(), vc[:, pos].contiguous())])
+    assert not np.isnan(got[0][0]).any()
+    for narrow, w in zip(*got):
+        assert np.array_equal(narrow, w)
+
+
 # ---- residual steps (model.py:775-788; model.cpp:409-420) ---------------------------
 
 @pytest.mark.parametrize("mode,norm_y,norm_out,K,pad", [(0, True, True, 3840, 4096), (1, True, False, 3840, 4096),
