@@ -53,6 +53,7 @@ extern "C" int alv_chain_run(const alv_chain_op* ops, int n, int M, void* stream
             if (int rc = launch_gemv(two[0], s)) return rc;
             if (int rc = launch_gemv(two[1], s)) return rc;
             c.ffn->last_a = c.ffn->a;
+            c.ffn->a_packed = false;
             c.ffn->a_rows = M;
         }
     }

@@ -18,9 +18,9 @@
 //   2. down = Wd * a, with a single bf16 term per activation value (it is
 //      bf16 by construction), summed entirely on the device -- the reference
 //      sums per-core partials on the host (runtime/cpp/src/npu.cpp:360-377).
-// Prefill (from 17 bf16 / 33 fp32 tokens): the same two steps with the MFMA
-// tiled kernel (gemm_q.hip);
-// the M x I activation lives in the stream's prefill scratch (q4_host.h).
+// Prefill (from 17 bf16 / 33 fp32 tokens): the same two steps with the prefill
+// kernel (prefill_q.hip); the M x I activation lives in the stream's scratch
+// (q4_host.h), in the down product's operand order.
 #include <stdlib.h>
 #include <string.h>
 
@@ -106,6 +106,38 @@ void ffn_ops(alv_ffn_t w, uint16_t* act, const float* X, int ldx, float* Y, int 
     down.Nz = w->H;
     down.parts = 1;
     down.tiled = true;
+}
+
+// The two launches of a prefill-sized call. The activation goes to the stream's
+// scratch; the handle's decode buffer keeps its size and address (graphs may
+// hold it). It is held in the down product's operand order, or, where the
+// prefill kernel does not take the call, row-major.
+static int ffn_prefill(alv_ffn_t w, GemvLaunch (&op)[2], hipStream_t s) {
+    const int M = op[0].M;
+    void* act = nullptr;
+    const size_t row_major = (size_t)M * w->I * sizeof(uint16_t);
+    if (int rc = get_scratch(s, kScratchAct, std::max(row_major, packed_bytes(M, w->Ie)), &act)) return rc;
+    op[0].Yb = nullptr;
+    op[0].Yp = static_cast<uint8_t*>(act);
+    bool taken = false;
+    if (int rc = launch_prefill(op[0], s, &taken)) return rc;
+    if (taken) {
+        op[1].Xb = nullptr;
+        op[1].Xp = static_cast<uint8_t*>(act);
+        if (int rc = launch_prefill(op[1], s, &taken)) return rc;
+        if (!taken) return fail(ALV_ERR_RANGE, "the down product of %d tokens is outside the prefill ranges", M);
+        if (int rc = launch_zero_rows(op[1], s)) return rc;
+    } else {
+        op[0].Yp = nullptr;
+        op[0].Yb = static_cast<uint16_t*>(act);
+        op[1].Xb = static_cast<uint16_t*>(act);
+        if (int rc = launch_gemm_tiled(op[0], s)) return rc;
+        if (int rc = launch_gemm_tiled(op[1], s)) return rc;
+    }
+    w->last_a = static_cast<uint16_t*>(act);
+    w->a_rows = M;
+    w->a_packed = taken;
+    return ALV_OK;
 }
 
 }  // namespace alv
@@ -212,17 +244,9 @@ extern "C" int alv_ffn_fused(alv_ffn_t w, const float* X, float* Y, int M, int l
     if (dev != w->device) return fail(ALV_ERR_HANDLE, "FFN handle belongs to device %d, current device is %d", w->device, dev);
     hipStream_t s = (hipStream_t)stream;
     if (M >= tiled_min_m(true)) {
-        // Prefill: the activation goes to the stream's scratch; the handle's
-        // decode buffer keeps its size and address (graphs may hold it).
-        void* act = nullptr;
-        if (int rc = get_scratch(s, kScratchAct, (size_t)M * w->I * sizeof(uint16_t), &act)) return rc;
         GemvLaunch op[2];
-        ffn_ops(w, static_cast<uint16_t*>(act), X, ldx, Y, ldy, M, op);
-        if (int rc = launch_gemm_tiled(op[0], s)) return rc;
-        if (int rc = launch_gemm_tiled(op[1], s)) return rc;
-        w->last_a = static_cast<uint16_t*>(act);
-        w->a_rows = M;
-        return ALV_OK;
+        ffn_ops(w, nullptr, X, ldx, Y, ldy, M, op);
+        return ffn_prefill(w, op, s);
     }
     if (M == 1 && w->vdown && ffn1_on()) {
         GemvLaunch op[2];
@@ -230,6 +254,7 @@ extern "C" int alv_ffn_fused(alv_ffn_t w, const float* X, float* Y, int M, int l
         if (int rc = launch_ffn1(op[0], w->vdown, w->vdown_bytes, w->part1, w->a, w->G1, w->U1, w->H, Y, nullptr, s))
             return rc;
         w->last_a = w->a;
+        w->a_packed = false;
         w->a_rows = 1;
         return ALV_OK;
     }
@@ -240,6 +265,7 @@ extern "C" int alv_ffn_fused(alv_ffn_t w, const float* X, float* Y, int M, int l
         if (int rc = launch_gemv(op[0], s)) return rc;
         if (int rc = launch_gemv(op[1], s)) return rc;
         w->last_a = w->a;
+        w->a_packed = false;
         w->a_rows = mc;
     }
     return ALV_OK;
@@ -265,16 +291,10 @@ extern "C" int alv_ffn_fused_bf16(alv_ffn_t w, const uint16_t* X, uint16_t* Y, i
         op[1].Yb = y;
     };
     if (M >= tiled_min_m(false)) {
-        void* act = nullptr;
-        if (int rc = get_scratch(s, kScratchAct, (size_t)M * w->I * sizeof(uint16_t), &act)) return rc;
         GemvLaunch op[2];
-        ffn_ops(w, static_cast<uint16_t*>(act), nullptr, ldx, nullptr, ldy, M, op);
+        ffn_ops(w, nullptr, nullptr, ldx, nullptr, ldy, M, op);
         bf16_ends(op, X, Y);
-        if (int rc = launch_gemm_tiled(op[0], s)) return rc;
-        if (int rc = launch_gemm_tiled(op[1], s)) return rc;
-        w->last_a = static_cast<uint16_t*>(act);
-        w->a_rows = M;
-        return ALV_OK;
+        return ffn_prefill(w, op, s);
     }
     if (M == 1 && w->vdown && ffn1_on()) {
         GemvLaunch op[2];
@@ -283,6 +303,7 @@ extern "C" int alv_ffn_fused_bf16(alv_ffn_t w, const uint16_t* X, uint16_t* Y, i
         if (int rc = launch_ffn1(op[0], w->vdown, w->vdown_bytes, w->part1, w->a, w->G1, w->U1, w->H, nullptr, Y, s))
             return rc;
         w->last_a = w->a;
+        w->a_packed = false;
         w->a_rows = 1;
         return ALV_OK;
     }
@@ -294,6 +315,7 @@ extern "C" int alv_ffn_fused_bf16(alv_ffn_t w, const uint16_t* X, uint16_t* Y, i
         if (int rc = launch_gemv(op[0], s)) return rc;
         if (int rc = launch_gemv(op[1], s)) return rc;
         w->last_a = w->a;
+        w->a_packed = false;
         w->a_rows = mc;
     }
     return ALV_OK;
@@ -374,12 +396,14 @@ extern "C" int alv_ffn_fused_bf16_addnorm(alv_ffn_t w, const uint16_t* resid, co
         if (int rc = launch_ffn1(op[0], w->vdown, w->vdown_bytes, w->part1, w->a, w->G1, w->U1, w->H, nullptr, Y, s))
             return rc;
         w->last_a = w->a;
+        w->a_packed = false;
         w->a_rows = 1;
         return ALV_OK;
     }
     if (int rc = launch_gemv(op[0], s)) return rc;
     if (int rc = launch_gemv(op[1], s)) return rc;
     w->last_a = w->a;
+    w->a_packed = false;
     w->a_rows = 1;
     return ALV_OK;
 }
@@ -404,6 +428,7 @@ extern "C" int alv_ffn_fused_noalloc(alv_ffn_t w, const float* X, float* Y, int 
                                  (hipStream_t)stream))
             return rc;
         w->last_a = w->a;
+        w->a_packed = false;
         w->a_rows = 1;
         return ALV_OK;
     }
@@ -422,6 +447,7 @@ extern "C" int alv_ffn_fused_noalloc(alv_ffn_t w, const float* X, float* Y, int 
         if (int rc = launch_gemv(L, s)) return rc;
     }
     w->last_a = w->a;
+    w->a_packed = false;
     w->a_rows = M;
     return ALV_OK;
 }
@@ -438,6 +464,7 @@ extern "C" int alv_ffn_gate_up(alv_ffn_t w, const float* X, int M, int ldx, void
     ffn_ops(w, w->a, X, ldx, nullptr, w->H, M, op);
     if (int rc = launch_gemv(op[0], (hipStream_t)stream)) return rc;
     w->last_a = w->a;
+    w->a_packed = false;
     w->a_rows = M;
     return ALV_OK;
 }
@@ -460,6 +487,7 @@ extern "C" int alv_ffn_partials(alv_ffn_t w, const float* X, float* P, int* slic
                              nullptr, (hipStream_t)stream, false))
         return rc;
     w->last_a = w->a;
+    w->a_packed = false;
     w->a_rows = 1;
     return ALV_OK;
 }
@@ -477,6 +505,8 @@ extern "C" int alv_ffn_activation(alv_ffn_t w, float* out, int M, void* stream) 
     if (int rc = check_handle(w)) return rc;
     if (!out) return fail(ALV_ERR_ARG, "null output pointer");
     if (M < 1 || M > w->a_rows) return fail(ALV_ERR_ARG, "M=%d outside the %d tokens of the last call", M, w->a_rows);
+    if (w->a_packed)
+        return launch_unpack_f32(reinterpret_cast<const uint8_t*>(w->last_a), M, w->Ie, out, w->I, (hipStream_t)stream);
     const int64_t n = (int64_t)M * w->I;
     const int grid = (int)std::min<int64_t>((n + 255) / 256, 4096);
     hipLaunchKernelGGL(bf16_to_f32_kernel, dim3(grid), dim3(256), 0, (hipStream_t)stream, w->last_a, out, n);

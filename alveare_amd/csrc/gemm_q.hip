@@ -1,6 +1,7 @@
-// MFMA Q4 GEMM for prefill-sized batches (gfx950): the path of alv_gemm_q,
-// alv_gemv, alv_gemv_bf16, alv_ffn_fused and alv_ffn_fused_bf16 from 17 (bf16
-// activations) or 33 (fp32) tokens (gate/up with the GLU epilogue, then down).
+// MFMA Q4 GEMM for prefill-sized batches (gfx950) on weights in the combined
+// layout: the path of alv_gemv_q and alv_gemm_q from 33 tokens. Registered
+// weights take prefill_q.hip, and this kernel only where that one's scratch
+// would have to grow during a graph capture or an operand is outside its ranges.
 //
 // C[M, N] = X[M, K] * dequant(W)[N, K]^T. A workgroup of 8 waves owns a
 // TM-token x 128-weight-row tile -- TM = 256, or 64 up to 128 tokens (a
@@ -481,6 +482,11 @@ hipError_t launch_gemm_x(const GemmArgs& a, bool xf32, int tm, dim3 grid, hipStr
 }  // namespace
 
 int launch_gemm_tiled(const GemvLaunch& L, hipStream_t s) {
+    if (L.tiled && !L.glu) {
+        bool taken = false;
+        if (int rc = launch_prefill(L, s, &taken)) return rc;
+        if (taken) return launch_zero_rows(L, s);
+    }
     const uint64_t wbytes = L.tiled ? tile_bytes(L.N, L.K) : (uint64_t)L.N * (uint64_t)(L.K / 32) * kBlockBytes;
     // Lane offset + step offset of a load must not wrap 32 bits: weights below
     // 3.75 GiB, activations below 2 GiB.
@@ -575,13 +581,15 @@ int launch_gemm_tiled(const GemvLaunch& L, hipStream_t s) {
     else
         e = L.tiled ? launch_gemm_x<1, true>(a, xf32, TM, grid, s) : launch_gemm_x<1, false>(a, xf32, TM, grid, s);
     if (int rc = hip_check(e, "gemm_q4_kernel launch")) return rc;
-    if (L.Nz > L.N) {
-        const int64_t n = (int64_t)(L.Nz - L.N) * L.M;
-        const int zg = (int)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 1024));
-        hipLaunchKernelGGL(zero_rows_kernel, dim3(zg), dim3(256), 0, s, L.Y, L.Yb, L.ldy, L.M, L.N, L.Nz);
-        return hip_check(hipGetLastError(), "zero_rows_kernel launch");
-    }
-    return ALV_OK;
+    return launch_zero_rows(L, s);
+}
+
+int launch_zero_rows(const GemvLaunch& L, hipStream_t s) {
+    if (L.Nz <= L.N || L.Yp) return ALV_OK;
+    const int64_t n = (int64_t)(L.Nz - L.N) * L.M;
+    const int zg = (int)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 1024));
+    hipLaunchKernelGGL(zero_rows_kernel, dim3(zg), dim3(256), 0, s, L.Y, L.Yb, L.ldy, L.M, L.N, L.Nz);
+    return hip_check(hipGetLastError(), "zero_rows_kernel launch");
 }
 
 }  // namespace alv

@@ -302,6 +302,25 @@ __device__ __forceinline__ bool glu_fast(float g, float u, int act, float* out) 
     return mag >= 0x04000000u && mag < 0x7E800000u && (b & 0xFFFFu) - 0x7FC0u > 0x80u;
 }
 
+// The GELU fast path in fewer instructions (prefill_q.hip: a tile's epilogue
+// evaluates 128 values per lane): z's factor, -2 and log2(e) are one constant c
+// and the hardware's exp2 and reciprocal take the place of expf and the
+// division. t = c inner: c and the product round by 1.5 * 2^-24 of |t| <= 31.8,
+// 33.1 * 2^-24 through 2^t; exp2 and the reciprocal 1 ulp each (2 * 2^-24),
+// the add and the two products 2^-24 each, and the reference's own 4 * 2^-24:
+// 45 fp32 ulps of v at most, against the 64 of the midpoint test.
+__device__ __forceinline__ bool gelu_quick(float g, float u, float* out) {
+#pragma clang fp contract(off)
+    const float g3 = (g * g) * g;
+    const float inner = g + 0.044715f * g3;
+    const float t = -2.3022081986f * inner;  // -2 sqrt(2 / pi) log2(e)
+    const float v = (g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t))) * u;
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const uint32_t mag = b & 0x7FFFFFFFu;
+    *out = v;
+    return t <= 31.7f && mag >= 0x04000000u && mag < 0x7E800000u && (b & 0xFFFFu) - 0x7FC0u > 0x80u;
+}
+
 // Fast path, else the float64 one: the prefill GEMM's epilogue (64 values
 // per lane) and alv_glu. The decode kernels evaluate a few values per lane,
 // where a wave that has any lane on the float64 path runs both paths, so they

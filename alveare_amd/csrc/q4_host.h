@@ -107,6 +107,11 @@ struct GemvLaunch {
     // Output rows [N, Nz) of every token are written as zeros (the all-zero
     // trailing rows a registration trimmed off, see weight_extent); Nz <= N: none.
     int Nz = 0;
+    // Prefill (launch_prefill): activations already in operand order (bf16,
+    // one term) in place of X / Xb, and the GLU's output in that order in
+    // place of Yb.
+    const uint8_t* Xp = nullptr;
+    uint8_t* Yp = nullptr;
 };
 int launch_gemv(const GemvLaunch& L, hipStream_t s);
 // The split-K partial-sum bytes launch_gemv(L) needs (0: no launch splits K),
@@ -135,6 +140,17 @@ constexpr int kGemvMaxM = 16;
 // MFMA tiled kernel for prefill-sized M (gemm_q.hip). Same contract as
 // GemvLaunch (glu pairs W0/W1 into the activation).
 int launch_gemm_tiled(const GemvLaunch& L, hipStream_t s);
+
+// The same product with the weights dequantized into operand registers and the
+// activations packed in operand order (prefill_q.hip); registered weights
+// only. *taken false (and nothing enqueued): the shape is outside its ranges,
+// or its scratch would have to grow during a graph capture.
+int launch_prefill(const GemvLaunch& L, hipStream_t s, bool* taken);
+// Bytes of M x K bf16 activations in operand order, and their widening to
+// row-major fp32 (columns K .. ldo - 1 zeros; K and ldo multiples of 8).
+size_t packed_bytes(int M, int K);
+int launch_unpack_f32(const uint8_t* in, int M, int K, float* out, int ldo, hipStream_t s);
+int launch_zero_rows(const GemvLaunch& L, hipStream_t s);
 
 // M at and above which the tiled kernel runs a product (below it the
 // streaming kernel, 16 tokens per launch), by activation type: bf16
@@ -212,6 +228,7 @@ struct alv_ffn {
     size_t a_cap;
     const uint16_t* last_a;  // activation of the last call: `a`, or the stream's prefill scratch
     int a_rows;              // tokens held at last_a after the last call
+    bool a_packed;           // last_a is in the prefill kernel's operand order (prefill_q.hip), Ie columns
     // One-token FFN in one launch (q4_ffn1_kernel; null vdown: the shape does
     // not take it): the down matrix again in slice order, and G x He partials.
     uint8_t* vdown;

@@ -1,0 +1,168 @@
+"""The prefill kernel (csrc/prefill_q.hip) at the edges of its tiles: token and
+row remainders, partial super-steps of K, every tile and K split its plan picks,
+one and three activation terms, the GLU epilogue's bits, and the scratch it
+keeps between calls."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(msg):
+    print(f"\n[prefill] {msg}", flush=True)
+
+
+def _weight(orc, dev, N, K, seed):
+    """A registered projection and its dequantized matrix in float64 (the
+    dequantization itself is pinned bit for bit by test_gpu_parity.py)."""
+    import alveare_amd as aa
+
+    W = torch.from_numpy(orc.synth_q4(N, K, seed)).to(dev)
+    return aa.Q4Weight(W, N, K), aa.dequant_q4(W, N, K).double()
+
+
+# tile (16-token blocks x 16-row blocks per wave) and split the plan picks: 2x2;
+# 2x2, two blocks; 4x2 split twice; 2x2 split 8 times (30 whole super-steps);
+# 4x2 split 8 times; 8x4, ragged rows; 12x4; 16x4, ragged tokens and rows.
+SHAPES = [(17, 333, 480), (31, 1000, 32), (600, 2000, 3872), (70, 512, 15360), (600, 544, 15360), (193, 30001, 544),
+          (300, 30720, 1024), (490, 30000, 1056)]
+
+
+# (fp32 activations take the streaming kernel below 33 tokens)
+@pytest.mark.parametrize("M,N,K,dtype", [(*s, d) for s in SHAPES for d in ("bf16", "fp32") if d == "bf16" or s[0] > 32])
+def test_prefill_products(orc, dev, M, N, K, dtype):
+    """Within the float32 bound of the float64 product: K + 8 roundings of 2^-24
+    over sum |x w| (three terms: 3 K + 8), a bf16 result half a bf16 ulp more
+    (2^-8 of the value: eight significant bits)."""
+    from alveare_amd import layer
+
+    _say(f"product M={M} N={N} K={K} {dtype}")
+    w, w64 = _weight(orc, dev, N, K, M + N)
+    x = torch.from_numpy(orc.synth_normal(M * K, M + K)).to(dev).view(M, K)
+    x = x.to(torch.bfloat16) if dtype == "bf16" else x
+    y = layer.gemv_bf16(w, x, M=M).view(M, N) if dtype == "bf16" else w(x, M=M)
+    x64 = x.double()
+    ref = x64 @ w64.T
+    bound = ((3 if dtype == "fp32" else 1) * K + 8) * 2.0 ** -24 * (x64.abs() @ w64.abs().T) + 1e-30
+    if dtype == "bf16":
+        bound = bound * 1.01 + ref.abs() * 2.0 ** -8
+    bad = ((y.double() - ref).abs() > bound).sum().item()
+    assert bad == 0, f"{bad} of {M * N} outside the float32 bound"
+    w.close()
+
+
+def _picker(I, H, cols):
+    """Combined-layout rows whose only nonzero weight is 1 at column cols[i]."""
+    W = np.zeros((I, H // 32, 20), np.uint8)
+    W[:, :, 17] = 0x3F  # bf16 1.0
+    W[:, :, 16] = 0x80
+    c = np.asarray(cols)
+    W[np.arange(I), c // 32, (c % 32) // 2] = np.where(c % 2, 0x10, 0x01)
+    return W.reshape(I, -1)
+
+
+@pytest.mark.parametrize("act", ["gelu", "silu"])
+@pytest.mark.parametrize("M,I", [(480, 15360), (330, 2080), (17, 2080)])
+def test_prefill_glu_bits(orc, dev, M, I, act):
+    """The epilogue's GLU gives alv_glu's bits (pinned to the reference by
+    test_glu_bit_exact) for M x I pairs: gate and up rows that pick one
+    activation each. Values over the float32 path's range, its edges and the
+    queue's: |g| from subnormal to 60, zeros, and a token of equal pairs next to
+    a rounding midpoint in every column."""
+    import alveare_amd as aa
+
+    _say(f"GLU bits M={M} I={I} {act}")
+    H, half = 1056, 528
+    rows = np.arange(I)
+    ffn = aa.pack_ffn_fused_weights(_picker(I, H, rows % half), _picker(I, H, half + rows // half),
+                                    orc.synth_q4(H, I, 5), H, I, activation=act, device=dev)
+    g = torch.Generator().manual_seed(M + I)
+    x = torch.randn(M, H, generator=g) * torch.exp2(torch.randint(-12, 6, (M, H), generator=g).float())
+    x[0] = 0.0
+    x[1, :half] = torch.linspace(-12.0, 12.0, half)
+    x[2, :half] = -torch.exp2(torch.linspace(-130.0, 5.9, half))
+    x[3] = 1.0  # one pair in every column
+    x = x.to(torch.bfloat16).to(dev)
+    y = torch.empty(M, H, dtype=torch.bfloat16, device=dev)
+    from alveare_amd import layer
+    layer.ffn_fused_bf16(ffn, x, y, M)
+    got = ffn.last_activation(M)
+    cols = torch.from_numpy(rows).to(dev)
+    gg = x.float()[:, cols % half].contiguous()
+    uu = x.float()[:, half + cols // half].contiguous()
+    want = torch.empty_like(gg)
+    aa._lib.check(aa.lib().alv_glu(gg.data_ptr(), uu.data_ptr(), want.data_ptr(), gg.numel(),
+                                   0 if act == "gelu" else 1, torch.cuda.current_stream().cuda_stream), "alv_glu")
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+    # and the down product of that activation
+    w64 = aa.dequant_q4(torch.from_numpy(orc.synth_q4(H, I, 5)).to(dev), H, I).double()
+    ref = got.double() @ w64.T
+    bound = (I + 8) * 2.0 ** -24 * (got.double().abs() @ w64.abs().T) + ref.abs() * 2.0 ** -8 + 1e-30
+    assert ((y.double() - ref).abs() <= 1.01 * bound).all()
+    ffn.close()
+
+
+def test_prefill_scratch_holds_no_old_values(orc, dev):
+    """A call whose packed activation is padded (35 blocks of 32: a last
+    substep of three) right after one that filled the stream's scratch with NaN."""
+    import alveare_amd as aa
+    from alveare_amd import layer
+
+    _say("padding after a NaN call")
+    big = aa.pack_ffn_fused_weights(orc.synth_q4(2048, 512, 1), orc.synth_q4(2048, 512, 2), orc.synth_q4(512, 2048, 3),
+                                    512, 2048, device=dev)
+    layer.ffn_fused_bf16(big, torch.full((200, 512), float("nan"), dtype=torch.bfloat16, device=dev), M=200)
+    H, I, M = 672, 1120, 45
+    Wg, Wu, Wd = orc.synth_q4(I, H, 4), orc.synth_q4(I, H, 5), orc.synth_q4(H, I, 6)
+    ffn = aa.pack_ffn_fused_weights(Wg, Wu, Wd, H, I, device=dev)
+    x = torch.from_numpy(orc.synth_normal(M * H, 7)).to(dev).view(M, H).to(torch.bfloat16)
+    y = layer.ffn_fused_bf16(ffn, x, M=M).view(M, H)
+    a = ffn.last_activation(M)
+    assert torch.isfinite(a).all()
+    ref = a.double() @ aa.dequant_q4(torch.from_numpy(Wd).to(dev), H, I).double().T
+    assert (y.double() - ref).abs().max() <= 2.0 ** -8 * ref.abs().max()
+    big.close()
+    ffn.close()
+
+
+def test_prefill_capture(orc, dev):
+    """Captured after an eager call of its shape, the packed path replays its
+    bits, eager work of other shapes between the replays; captured on a stream
+    whose scratch was never sized, the call still runs (the kernel that needs
+    no scratch) and agrees within bf16 rounding of the same sums."""
+    from alveare_amd import layer
+
+    _say("capture")
+    M, N, K = 45, 700, 1056
+    w, w64 = _weight(orc, dev, N, K, 11)
+    x = torch.from_numpy(orc.synth_normal(M * K, 12)).to(dev).view(M, K).to(torch.bfloat16)
+    other = torch.from_numpy(orc.synth_normal(300 * K, 13)).to(dev).view(300, K).to(torch.bfloat16)
+    want = layer.gemv_bf16(w, x, M=M).clone()
+    ref = x.double() @ w64.T
+    bound = (K + 8) * 2.0 ** -24 * (x.double().abs() @ w64.abs().T) * 1.01 + ref.abs() * 2.0 ** -8
+    for sized in (True, False):
+        s = torch.cuda.Stream(device=dev)
+        y = torch.empty(M * N, dtype=torch.bfloat16, device=dev)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            if sized:
+                layer.gemv_bf16(w, x, y, M)
+            s.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=s):
+                layer.gemv_bf16(w, x, y, M)
+            for _ in range(3):
+                y.zero_()
+                graph.replay()
+                s.synchronize()
+                if sized:
+                    assert torch.equal(y, want)
+                assert ((y.view(M, N).double() - ref).abs() <= bound).all()
+                if sized:
+                    layer.gemv_bf16(w, other, M=300)
+                s.synchronize()
+    w.close()
