@@ -34,7 +34,7 @@ import torch
 from ._lib import check, lib
 import math
 
-from .ops import FfnWeights, Q4Weight, _need_gpu, _stream, lm_head
+from .ops import FfnWeights, Q4Weight, _need_gpu, _on, _stream, lm_head
 
 _GEMMA_EPS = 1e-6
 
@@ -52,7 +52,8 @@ def _bf16(t: torch.Tensor, name: str, n: int) -> torch.Tensor:
 def _f32(t, name: str, n: int, dev) -> torch.Tensor | None:
     if t is None:
         return None
-    t = torch.as_tensor(t, dtype=torch.float32, device=dev).contiguous()
+    if not (isinstance(t, torch.Tensor) and t.dtype == torch.float32 and t.device == dev and t.is_contiguous()):
+        t = torch.as_tensor(t, dtype=torch.float32, device=dev).contiguous()
     if t.numel() < n:
         raise ValueError(f"{name} has {t.numel()} elements, needs {n}")
     return t
@@ -74,7 +75,7 @@ def rmsnorm(x: torch.Tensor, w=None, *, K: int | None = None, rows: int = 1, pad
     if out is None:
         out = torch.empty(rows * pad, dtype=torch.bfloat16, device=dev)
     _bf16(out, "out", rows * pad)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check(lib().alv_rmsnorm(x.data_ptr(), _ptr(w), out.data_ptr(), rows, K, K, pad, pad, ctypes.c_float(eps),
                                 _stream(x)), "alv_rmsnorm")
     return out
@@ -109,7 +110,7 @@ def qkv_post(qkv: torch.Tensor, pos_dev: torch.Tensor, kcache: torch.Tensor, vca
     if q_out is None:
         q_out = torch.empty(heads * D, dtype=torch.bfloat16, device=dev)
     _bf16(q_out, "q_out", heads * D)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check(lib().alv_qkv_post(qkv.data_ptr(), k_off, v_off, heads, kv_heads, D, _ptr(q_w), _ptr(k_w), int(norm_q),
                                  int(norm_k), int(norm_v), ctypes.c_float(eps), _ptr(rope), rope_stride or 0, cos_off,
                                  sin_off or 0, half or 0, pos_dev.data_ptr(), kcache.shape[1], q_out.data_ptr(),
@@ -150,7 +151,7 @@ def qkv_attention(qkv: torch.Tensor, pos_dev: torch.Tensor, kcache: torch.Tensor
     if out is None:
         out = torch.empty(heads * D, dtype=torch.bfloat16, device=dev)
     _bf16(out, "out", heads * D)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check(lib().alv_qkv_attention(qkv.data_ptr(), k_off, v_off, heads, kv_heads, D, _ptr(q_w), _ptr(k_w),
                                       int(norm_q), int(norm_k), int(norm_v), ctypes.c_float(eps), _ptr(rope),
                                       rope_stride or 0, cos_off, sin_off or 0, half or 0, pos_dev.data_ptr(),
@@ -171,7 +172,7 @@ def attention(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, pos_d
     if out is None:
         out = torch.empty(heads * D, dtype=torch.bfloat16, device=dev)
     _bf16(out, "out", heads * D)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check(lib().alv_attention(q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), out.data_ptr(), heads, kv_heads,
                                   D, max_seq, window, ctypes.c_float(scale), pos_dev.data_ptr(), _stream(q)),
               "alv_attention")
@@ -197,7 +198,7 @@ def add_norm(resid: torch.Tensor, y: torch.Tensor, *, K: int, w_y=None, norm_y: 
         norm_buf = torch.empty(rows * pad, dtype=torch.bfloat16, device=dev)
     if norm_out:
         _bf16(norm_buf, "norm_out", rows * pad)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check(lib().alv_add_norm(resid.data_ptr(), K, y.data_ptr(), K, _ptr(w_y), int(norm_y), ctypes.c_float(scale),
                                  scale_mode, sum_out.data_ptr(), K, _ptr(w_out), _ptr(norm_buf) if norm_out else 0,
                                  pad, rows, K, pad, ctypes.c_float(eps), _stream(resid)), "alv_add_norm")
@@ -210,7 +211,7 @@ def gemv_bf16(W: Q4Weight, X: torch.Tensor, Y: torch.Tensor | None = None, M: in
     if Y is None:
         Y = torch.empty(M * W.N, dtype=torch.bfloat16, device=W.device)
     _bf16(Y, "Y", M * W.N)
-    with torch.cuda.device(W.device):
+    with _on(W.device):
         check(lib().alv_gemv_bf16(W.handle, X.data_ptr(), Y.data_ptr(), M, W.K, W.N, _stream(X)), "alv_gemv_bf16")
     return Y
 
@@ -221,7 +222,7 @@ def ffn_fused_bf16(F: FfnWeights, X: torch.Tensor, Y: torch.Tensor | None = None
     if Y is None:
         Y = torch.empty(M * F.H, dtype=torch.bfloat16, device=F.device)
     _bf16(Y, "Y", M * F.H)
-    with torch.cuda.device(F.device):
+    with _on(F.device):
         check(lib().alv_ffn_fused_bf16(F.handle, X.data_ptr(), Y.data_ptr(), M, F.H, F.H, _stream(X)),
               "alv_ffn_fused_bf16")
     return Y
@@ -258,7 +259,7 @@ def gemv_bf16_addnorm(W: Q4Weight, resid: torch.Tensor, y: torch.Tensor | None, 
     if Y is None:
         Y = torch.empty(W.N, dtype=torch.bfloat16, device=W.device)
     _bf16(Y, "Y", W.N)
-    with torch.cuda.device(W.device):
+    with _on(W.device):
         check(lib().alv_gemv_bf16_addnorm(W.handle, *args, Y.data_ptr(), _stream(resid)), "alv_gemv_bf16_addnorm")
     return Y
 
@@ -290,7 +291,7 @@ def lm_head_addnorm(W: Q4Weight, resid: torch.Tensor, y: torch.Tensor | None, *,
         raise TypeError("token must be an int32 tensor on the weights' device")
     if pos is not None and (pos.dtype != torch.int32 or pos.device != W.device or pos.numel() < 1):
         raise TypeError("pos must be an int32 tensor on the weights' device")
-    with torch.cuda.device(W.device):
+    with _on(W.device):
         check(lib().alv_lm_head_bf16_addnorm(W.handle, *args, int(hidden), logits.data_ptr(), vocab, float(softcap),
                                              token.data_ptr(), pos.data_ptr() if pos is not None else None,
                                              int(max_pos), _stream(resid)), "alv_lm_head_bf16_addnorm")
@@ -307,7 +308,7 @@ def ffn_fused_bf16_addnorm(F: FfnWeights, resid: torch.Tensor, y: torch.Tensor, 
     if Y is None:
         Y = torch.empty(F.H, dtype=torch.bfloat16, device=F.device)
     _bf16(Y, "Y", F.H)
-    with torch.cuda.device(F.device):
+    with _on(F.device):
         check(lib().alv_ffn_fused_bf16_addnorm(F.handle, *args, Y.data_ptr(), _stream(resid)),
               "alv_ffn_fused_bf16_addnorm")
     return Y
@@ -326,7 +327,7 @@ def embed(table: torch.Tensor, token_dev: torch.Tensor, scale: float, out: torch
     if out is None:
         out = torch.empty(H, dtype=torch.bfloat16, device=dev)
     _bf16(out, "out", H)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check(lib().alv_embed(table.data_ptr(), vocab, H, token_dev.data_ptr(), ctypes.c_double(scale), out.data_ptr(),
                               _stream(table)), "alv_embed")
     return out

@@ -36,7 +36,27 @@ _ACTS = {"gelu": ALV_ACT_GELU_TANH, "gelu_tanh": ALV_ACT_GELU_TANH, "silu": ALV_
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The raw handle of torch's current stream on t's device
+    (``torch.cuda.current_stream`` builds a Stream object for it: 1.5 us of a
+    call that the kernel itself may take 5 of)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+class _SameDevice:
+    def __enter__(self):
+        pass
+
+    def __exit__(self, *exc):
+        return False
+
+
+_SAME = _SameDevice()
+
+
+def _on(dev: torch.device):
+    """``torch.cuda.device(dev)``, or nothing to enter when dev is the current
+    device already (the switch and back took 2.5 us per call)."""
+    return _SAME if torch._C._cuda_getDevice() == dev.index else torch.cuda.device(dev)
 
 
 def _need_gpu(*ts: torch.Tensor) -> torch.device:
@@ -88,6 +108,8 @@ def _weight(W: torch.Tensor, N: int, K: int, name: str = "W") -> torch.Tensor:
 
 def _act_in(X: torch.Tensor, n: int, name: str) -> torch.Tensor:
     _too_small(name, X.numel(), n)
+    if X.dtype == torch.float32 and X.is_contiguous():
+        return X  # used by its address alone
     X = X.reshape(-1)[:n]
     if X.dtype == torch.bfloat16:
         X = X.float()
@@ -102,6 +124,8 @@ def _check_shape(N: int, K: int) -> None:
 
 
 def _store(Y: torch.Tensor, y32: torch.Tensor, n: int) -> None:
+    if y32 is Y:
+        return
     flat = Y.view(-1)
     if flat.data_ptr() == y32.data_ptr():
         return
@@ -111,7 +135,7 @@ def _store(Y: torch.Tensor, y32: torch.Tensor, n: int) -> None:
 def _out_buffer(Y: torch.Tensor, n: int, name: str) -> torch.Tensor:
     _too_small(name, Y.numel(), n)
     if Y.dtype == torch.float32 and Y.is_contiguous():
-        return Y.view(-1)[:n]
+        return Y
     if Y.dtype not in (torch.float32, torch.bfloat16):
         raise TypeError(f"{name} must be float32 or bfloat16, got {Y.dtype}")
     return torch.empty(n, dtype=torch.float32, device=Y.device)
@@ -125,7 +149,7 @@ def gemv_q(W: torch.Tensor, X: torch.Tensor, Y: torch.Tensor, *, N: int, K: int,
     W = _weight(W, N, K)
     x = _act_in(X, K, "X")
     y = _out_buffer(Y, N, "Y")
-    with torch.cuda.device(W.device):
+    with _on(W.device):
         check(lib().alv_gemv_q(W.data_ptr(), x.data_ptr(), y.data_ptr(), N, K, _stream(W)), "alv_gemv_q")
     _store(Y, y, N)
     return Y
@@ -141,7 +165,7 @@ def gemm_q(W: torch.Tensor, X: torch.Tensor, Y: torch.Tensor, *, B: int, N: int,
     W = _weight(W, N, K)
     x = _act_in(X, B * K, "X")
     y = _out_buffer(Y, B * N, "Y")
-    with torch.cuda.device(W.device):
+    with _on(W.device):
         check(lib().alv_gemm_q(W.data_ptr(), x.data_ptr(), y.data_ptr(), B, N, K, K, N, _stream(W)),
               "alv_gemm_q")
     _store(Y, y, B * N)
@@ -154,7 +178,7 @@ def dequant_q4(W: torch.Tensor, N: int, K: int) -> torch.Tensor:
     _need_gpu(W)
     W = _weight(W, N, K)
     out = torch.empty((N, K), dtype=torch.bfloat16, device=W.device)
-    with torch.cuda.device(W.device):
+    with _on(W.device):
         check(lib().alv_dequant_q4(W.data_ptr(), out.data_ptr(), N, K, _stream(W)), "alv_dequant_q4")
     return out
 
@@ -166,7 +190,7 @@ def q4_tile(W: torch.Tensor, N: int, K: int) -> torch.Tensor:
     _need_gpu(W)
     W = _weight(W, N, K)
     out = torch.empty(int(lib().alv_q4_tiled_bytes(N, K)), dtype=torch.uint8, device=W.device)
-    with torch.cuda.device(W.device):
+    with _on(W.device):
         check(lib().alv_q4_tile(W.data_ptr(), out.data_ptr(), N, K, _stream(W)), "alv_q4_tile")
     return out
 
@@ -192,7 +216,7 @@ def quantize_q4(W: torch.Tensor, N: int | None = None, K: int | None = None) -> 
     as quantize_and_pack_tensor does (tools/quantize_gemma4.py:26-41)."""
     W, n_src, k_src, N, K = _float_source(W, N, K)
     out = torch.empty((N, K // 32 * 20), dtype=torch.uint8, device=W.device)
-    with torch.cuda.device(W.device):
+    with _on(W.device):
         check(lib().alv_quantize_q4(W.data_ptr(), n_src, k_src, W.stride(0), out.data_ptr(), N, K, _stream(W)),
               "alv_quantize_q4")
     return out
@@ -211,7 +235,7 @@ class Q4Weight:
         self = cls.__new__(cls)
         self.N, self.K, self.device = N, K, W.device
         self._h = ctypes.c_void_p()
-        with torch.cuda.device(W.device):
+        with _on(W.device):
             check(lib().alv_weight_quantize(W.data_ptr(), n_src, k_src, W.stride(0), N, K, ctypes.byref(self._h),
                                             _stream(W)), "alv_weight_quantize")
         self.shape = (N, K // 32 * 20)
@@ -223,7 +247,7 @@ class Q4Weight:
         W = _weight(W, N, K)
         self.N, self.K, self.device = N, K, dev
         self._h = ctypes.c_void_p()
-        with torch.cuda.device(dev):
+        with _on(dev):
             check(lib().alv_weight_register(W.data_ptr(), N, K, ctypes.byref(self._h), _stream(W)),
                   "alv_weight_register")
         self.shape = (N, K // 32 * 20)
@@ -244,7 +268,7 @@ class Q4Weight:
 
     def close(self) -> None:
         if self._h:
-            with torch.cuda.device(self.device):
+            with _on(self.device):
                 lib().alv_weight_release(self._h)
             self._h = ctypes.c_void_p()
 
@@ -263,7 +287,7 @@ class Q4Weight:
             Y = torch.empty((M, self.N) if M > 1 else (self.N,), dtype=torch.float32, device=self.device)
         _need_gpu(Y)
         y = _out_buffer(Y, M * self.N, "Y")
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             check(lib().alv_gemv(self.handle, x.data_ptr(), y.data_ptr(), M, self.K, self.N, _stream(x)),
                   "alv_gemv")
         _store(Y, y, M * self.N)
@@ -288,7 +312,7 @@ class FfnWeights:
         w_down = _weight(w_down, H, I, "w_down")
         self.H, self.I, self.activation, self.device = H, I, activation, dev
         self._h = ctypes.c_void_p()
-        with torch.cuda.device(dev):
+        with _on(dev):
             check(lib().alv_ffn_register(w_gate.data_ptr(), w_up.data_ptr(), w_down.data_ptr(), H, I,
                                          _ACTS[activation], ctypes.byref(self._h), _stream(w_gate)),
                   "alv_ffn_register")
@@ -311,7 +335,7 @@ class FfnWeights:
 
     def close(self) -> None:
         if self._h:
-            with torch.cuda.device(self.device):
+            with _on(self.device):
                 lib().alv_ffn_release(self._h)
             self._h = ctypes.c_void_p()
 
@@ -324,7 +348,7 @@ class FfnWeights:
     def last_activation(self, M: int = 1) -> torch.Tensor:
         """The bf16-valued activation (M, I) of the last call (parity checks)."""
         out = torch.empty((M, self.I), dtype=torch.float32, device=self.device)
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             check(lib().alv_ffn_activation(self.handle, out.data_ptr(), M, _stream(out)),
                   "alv_ffn_activation")
         return out
@@ -335,7 +359,7 @@ class FfnWeights:
         x = _act_in(X, M * self.H, "X")
         if x.device != self.device:
             raise ValueError(f"X on {x.device}, weights on {self.device}")
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             check(lib().alv_ffn_gate_up(self.handle, x.data_ptr(), M, self.H, _stream(x)), "alv_ffn_gate_up")
 
     def partials(self, X: torch.Tensor, P: torch.Tensor | None = None) -> int:
@@ -347,7 +371,7 @@ class FfnWeights:
         if x.device != self.device:
             raise ValueError(f"X on {x.device}, weights on {self.device}")
         g = ctypes.c_int(0)
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             check(lib().alv_ffn_partials(self.handle, x.data_ptr(), P.data_ptr() if P is not None else None,
                                          ctypes.byref(g), _stream(x)), "alv_ffn_partials")
         return g.value
@@ -360,7 +384,7 @@ class FfnWeights:
             Y = torch.empty((M, self.H) if M > 1 else (self.H,), dtype=torch.float32, device=self.device)
         _need_gpu(Y)
         y = _out_buffer(Y, M * self.H, "Y")
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             check(lib().alv_ffn_fused(self.handle, x.data_ptr(), y.data_ptr(), M, self.H, self.H,
                                       _stream(x)), "alv_ffn_fused")
         _store(Y, y, M * self.H)
@@ -466,7 +490,7 @@ def lm_head(W: "Q4Weight", x: torch.Tensor, vocab: int | None = None, softcap: f
         raise TypeError("token must be an int32 tensor on the weights' device")
     if pos is not None and (pos.dtype != torch.int32 or pos.device != W.device or pos.numel() < 1):
         raise TypeError("pos must be an int32 tensor on the weights' device")
-    with torch.cuda.device(W.device):
+    with _on(W.device):
         if bf:
             check(lib().alv_lm_head_bf16(W.handle, xv.data_ptr(), logits.data_ptr(), vocab, float(softcap),
                                          token.data_ptr(), pos.data_ptr() if pos is not None else None,
