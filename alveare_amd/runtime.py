@@ -35,6 +35,7 @@ from pathlib import Path
 import numpy as np
 import torch
 
+from .layer import gemv_bf16
 from .ops import FfnWeights, Q4Weight, gemm_q, gemv_q, lm_head, pack_ffn_fused_weights
 
 PROJECTIONS = ["attn_q", "attn_k", "attn_v", "attn_output", "ffn_gate", "ffn_up", "ffn_down"]
@@ -198,6 +199,11 @@ class Q4Dispatch:
         if X.ndim != 2:
             raise ValueError("run_gemm_npu takes a (B, K) batch")
         B = X.shape[0]
+        if (isinstance(W_combined, ResidentWeight) and X.dtype == torch.bfloat16 and X.data_ptr() % 16 == 0
+                and X.device == rw.q4().device):
+            # bf16 in and out of the kernel: the float32 detour was three more
+            # launches and 10 bytes more per activation and result.
+            return self._out(gemv_bf16(rw.q4(), X, torch.empty((B, N), dtype=torch.bfloat16, device=X.device), B))
         Y = torch.empty((B, N), dtype=torch.float32, device=self.device)
         if isinstance(W_combined, ResidentWeight):
             rw.q4()(X.float(), Y, M=B)
