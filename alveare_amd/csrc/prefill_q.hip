@@ -6,9 +6,9 @@
 //   1. pack_x_kernel lays the activations out once in MFMA operand order
 //      (below), splitting fp32 values exactly into three bf16 terms; the FFN's
 //      gate/up launch writes its activation in that order itself.
-//   2. prefill_kernel: 4 waves per workgroup; a wave owns RB 16-row tiles of
-//      weights (for the GLU half gate, half up) against all TB x 16 tokens of
-//      the workgroup.
+//   2. prefill_kernel: 4 or 8 waves per workgroup; a wave owns RB = 2 16-row
+//      tiles of weights (for the GLU one gate, one up) against all TB x 16
+//      tokens of the workgroup.
 //
 // Weights never touch LDS: lane (g, j) of v_mfma_f32_16x16x32_bf16's B operand
 // holds 8 consecutive k of row j, one dword of nibbles, so each wave
@@ -21,12 +21,15 @@
 //
 // What bounds it: up to 128 tokens the dequantization (68 VALU clocks per 16 x
 // 32 weights a wave, as many as 4.25 matrix instructions) and the launches'
-// latency; above, the matrix cores at 1.1 PFLOP/s of the 1.45 that a large bf16
-// product reaches on this card (a 256 x 256 x 128 substep's matrix instructions
-// take 1.7 us and the substep 2.6: 84 KiB of operands per CU and substep from
-// the L2s, one wave per SIMD at the accumulators' size). FFN 3840 <-> 15360, bf16,
-// us per call, gemm_q.hip before and this kernel: 17 tokens 70 -> 51, 45: 72 -> 60,
-// 128: 111 -> 79, 200: 146 -> 115, 512: 207 -> 194, 1024: 392 -> 355, 3001: 1220 -> 954.
+// latency; above, LDS reads (every wave reads all of the workgroup's
+// activations, 512 KiB per 256 x 256 x 128 substep: 4096 clocks, as many as its
+// matrix instructions) at 1.1-1.2 PFLOP/s of the 1.45 that a large bf16 product
+// reaches on this card. Eight waves of two row tiles, two per SIMD, rather than
+// four of four: a wave alone on its SIMD does not overlap its dequantization
+// with its own matrix instructions (512 tokens 194 against 187 us, 3001: 954
+// against 912). FFN 3840 <-> 15360, bf16, us per call, gemm_q.hip before and
+// this kernel: 17 tokens 70 -> 51, 45: 72 -> 60, 128: 111 -> 82, 200: 146 -> 113,
+// 512: 207 -> 187, 3001: 1223 -> 912.
 //
 // The order of k. A super-step of the tiled layout (512 columns, 16 blocks) is
 // taken in T = 4 substeps of 128: substep t multiplies block T g + t in lane
@@ -187,9 +190,9 @@ __device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, uint32_t vo
 }
 
 // c += a b on the matrix cores. ACC: written out, with c in accumulation
-// registers, so that the result stays in c's own registers: with 128 or more
-// of them the compiler, left to choose, moved accumulators between register
-// files (420 moves per 256 of these) and spilled. It cannot see these writes'
+// registers, so that the result stays in c's own registers: with some 100 or
+// more of them the compiler, left to choose, moved accumulators between
+// register files (420 moves per 256 of these) and spilled. It cannot see these writes'
 // latency, so code that reads c otherwise first waits (acc_wait), and a and b
 // are written two instructions or more ahead.
 template <bool ACC>
@@ -234,21 +237,30 @@ struct Dequant {
 };
 constexpr int kDequantSteps = 17;
 
-// Substeps whose activations are loaded together: enough work (4096 clocks of
-// matrix instructions) for the next ones to arrive where a CU holds one
-// workgroup, one where several cover for each other.
+// Substeps whose activations are loaded together: enough work for the next
+// ones to arrive where a CU holds one workgroup (one substep of 8 x 16 tokens
+// is 2048 clocks of matrix instructions, about the latency of the L2 under this
+// load), one where several workgroups cover for each other.
 template <int TB>
 constexpr int prefill_stage() {
     return TB == 8 ? 2 : 1;
 }
 
+// Waves per workgroup: eight, two per SIMD, where a CU's LDS and registers hold
+// one such workgroup; four, several workgroups per CU, for small tiles.
+template <int TB, int RB>
+constexpr int prefill_wg() {
+    return TB >= 8 ? 8 : 4;
+}
+
 template <int TB, int RB>
 constexpr int prefill_waves() {  // waves per SIMD the register budget is set for
-    return TB * RB >= 32 ? 1 : TB * RB >= 16 ? 2 : 3;
+    return TB >= 8 ? 2 : 3;
 }
 
 template <int TB, int RB, bool GLU>
-__global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel(PrefillArgs a) {
+__global__ void __launch_bounds__((64 * prefill_wg<TB, RB>()), (prefill_waves<TB, RB>())) prefill_kernel(PrefillArgs a) {
+    constexpr int NWV = prefill_wg<TB, RB>(), NT = 64 * NWV;
     constexpr int RBM = GLU ? RB / 2 : RB;  // row tiles of one matrix per wave
     constexpr int PS = prefill_stage<TB>();      // substeps per stage: an LDS buffer, a barrier
     constexpr int BUF = PS * TB * kStepBytes;    // one LDS buffer
@@ -268,7 +280,7 @@ __global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel
     const int grp = idx / (4 * a.ty), rem = idx - grp * 4 * a.ty;
     const int gm = min(4, a.tx - 4 * grp);
     const int ty = rem / gm, tx = 4 * grp + rem - ty * gm;
-    const int m0 = tx * TB * 16, rt0 = ty * 4 * RBM + wave * RBM;
+    const int m0 = tx * TB * 16, rt0 = ty * NWV * RBM + wave * RBM;
 
     const PackGeom pg = a.pg;
     const __amdgpu_buffer_rsrc_t rw0 = make_rsrc(a.W0, a.wbytes);
@@ -288,7 +300,7 @@ __global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel
     if (a.flags) {
         const int nf = (min(m0 + TB * 16, a.M) - m0 + 15) / 16 * pg.nss;
         bool more = false;
-        for (int q = tid; q < nf; q += 256) more |= a.flags[(m0 >> 4) * pg.nss + q] != 0;
+        for (int q = tid; q < nf; q += NT) more |= a.flags[(m0 >> 4) * pg.nss + q] != 0;
         nterms = __syncthreads_or(more) ? 3 : 1;
     }
     // This split's whole super-steps [ss0, ss1), and the substeps of the last,
@@ -353,8 +365,9 @@ __global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel
     // other's latest loads), and the next substep's first octet follows. A
     // group is one row tile's dequantization between the matrix instructions
     // of G fragments.
-    constexpr int G = TB / RB, R = RB >= 4 ? 4 : 8 < 4 * TB ? 8 : 4 * TB;  // R: operand reads ahead
-    constexpr int LK = PS, LG = (PS * TB + LK * RB - 1) / (LK * RB);  // activation loads: over LK octets, per group
+    constexpr int G = TB / RB, R = RB >= 4 ? 4 : NWV == 8 ? 6 : 8 < 4 * TB ? 8 : 4 * TB;  // R: operand reads ahead
+    constexpr int XL = 4 * TB / NWV;  // fragments a wave loads per substep
+    constexpr int LK = PS, LG = (PS * XL + LK * RB - 1) / (LK * RB);  // activation loads: over LK octets, per group
     static_assert(TB % RB == 0, "whole fragments per group");
     auto substep = [&](auto tt, int s, int p, int nextss) __attribute__((always_inline)) {
         constexpr int TT = decltype(tt)::value;
@@ -391,8 +404,8 @@ __global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel
             for (int h = 0; h < RB; ++h) {
                 if (kk < LK && first)
 #pragma unroll
-                    for (int q = LG * (kk * RB + h); q < LG * (kk * RB + h + 1) && q < PS * TB; ++q)
-                        load_x(s + PS + q / TB, p, wave * TB + q % TB);
+                    for (int q = LG * (kk * RB + h); q < LG * (kk * RB + h + 1) && q < PS * XL; ++q)
+                        load_x(s + PS + q / XL, p, wave * XL + q % XL);
                 Dequant dq;
                 dq.d = kk < 3 ? dword(h, kk + 1) : TT == 4 ? wt[h][0] : dword(h, 5);
 #pragma unroll
@@ -400,7 +413,7 @@ __global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel
                     const int f = kk * TB + t;
 #pragma unroll
                     for (int q = 0; q < RB; ++q) {
-                        mfma_acc<(TB * RB >= 32)>(acc[t][q], av[f % R], bv[kk & 1][q]);
+                        mfma_acc<(TB * RB >= 24)>(acc[t][q], av[f % R], bv[kk & 1][q]);
                         const int slot = (t - G * h) * RB + q;
 #pragma unroll
                         for (int i = 0; i < kDequantSteps; ++i)
@@ -425,7 +438,7 @@ __global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel
     };
     for (int p = 0; p < nterms; ++p) {
 #pragma unroll
-        for (int q = 0; q < PS * TB; ++q) load_x(4 * ss0 + q / TB, p, wave * TB + q % TB);
+        for (int q = 0; q < PS * XL; ++q) load_x(4 * ss0 + q / XL, p, wave * XL + q % XL);
         if (ntail) load_tail(0, wt);
         if (ss0 < ss1) {
 #pragma unroll
@@ -456,12 +469,12 @@ __global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel
 
     // ---- split K: the last workgroup of the tile adds the partial tiles, in
     // split order (gemm_q.hip's scheme: 16-byte write-through pieces, thread
-    // tid's f32x4 (t, q) at ((t RB + q) 256 + tid) 16 bytes of its split).
+    // tid's f32x4 (t, q) at ((t RB + q) NT + tid) 16 bytes of its split).
     if (a.ks > 1) {
-        const size_t tsz = (size_t)TB * RB * 1024;  // floats of a tile
+        const size_t tsz = (size_t)TB * RB * NT * 4;  // floats of a tile
         const __amdgpu_buffer_rsrc_t rp = make_rsrc(a.part + (size_t)idx * a.ks * tsz, (uint32_t)(a.ks * tsz * sizeof(float)));
         auto piece = [&](int k, int t, int q) -> uint32_t {
-            return (uint32_t)((((size_t)k * TB + t) * RB + q) * 4096 + tid * 16);
+            return (uint32_t)((((size_t)k * TB + t) * RB + q) * (NT * 16) + tid * 16);
         };
 #pragma unroll
         for (int t = 0; t < TB; ++t)
@@ -498,7 +511,7 @@ __global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel
         // contiguous bytes). Values the float32 path cannot settle (about one
         // in 500) are queued and evaluated together: one by one where they
         // occur, nearly every octet's wave would run the float64 path.
-        constexpr int NR = 64 * RBM, LS = NR + 4;  // rows, LDS row stride in pairs
+        constexpr int NR = 16 * NWV * RBM, LS = NR + 4;  // rows, LDS row stride in pairs
         uint32_t* tile = reinterpret_cast<uint32_t*>(smem);
         __shared__ int queued, queue[kQueue];
         bool over = false;
@@ -517,7 +530,7 @@ __global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel
         const PackGeom po = pack_geom(a.N);
         const int n0 = ty * NR;
 #pragma unroll 1
-        for (int c = tid; c < TB * 16 * (NR / 8); c += 256) {
+        for (int c = tid; c < TB * 16 * (NR / 8); c += NT) {
             const int i = c & 15, o = (c >> 4) % (NR / 8), t = (c >> 4) / (NR / 8);
             const int m = m0 + 16 * t + i, n = n0 + 8 * o;
             if (m0 + 16 * t >= a.M || n >= a.N) continue;
@@ -555,7 +568,7 @@ __global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel
         const bool all = __syncthreads_or(over);
         const int nq = all ? TB * 16 * NR : queued;
 #pragma unroll 1
-        for (int c = tid; c < nq; c += 256) {
+        for (int c = tid; c < nq; c += NT) {
             const int at = all ? c / NR * LS + c % NR : queue[c];
             const int mt = at / LS, nt = at - mt * LS;
             if (m0 + mt >= a.M || n0 + nt >= a.N) continue;
@@ -567,7 +580,7 @@ __global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel
         // are, and what the buffer held before may not be finite.
         const int npad = 4 * po.T - po.nbl;
         if (ty == a.ty - 1)
-            for (int c = tid; c < TB * 64 * npad; c += 256) {
+            for (int c = tid; c < TB * 64 * npad; c += NT) {
                 const int i = c & 15, o = (c >> 4) % (4 * npad), t = (c >> 4) / (4 * npad);
                 if (m0 + 16 * t < a.M)
                     *reinterpret_cast<u32x4*>(a.Yp + pack_offset(po, m0 + 16 * t + i, a.N / 8 + o)) = u32x4{0, 0, 0, 0};
@@ -590,45 +603,46 @@ __global__ void __launch_bounds__(256, (prefill_waves<TB, RB>())) prefill_kernel
 }
 
 struct Plan {
-    int tb, rb, ks;
+    int tb, rb, waves, ks;
 };
 
 // Tile and K split of a product: the least estimated time over the tiles
 // built. A substep's time and a workgroup's own (prologue, epilogue) are fits,
-// in us, to sweeps of every tile and split over FFNs of 3840 <-> 15360, 1152 <->
+// in us, to sweeps of tiles (four-wave ones of 8, 12 and 16 blocks, within 10 %
+// of the eight-wave ones since) and splits over FFNs of 3840 <-> 15360, 1152 <->
 // 6912 and 1056 <-> 14400 at 17 to 3001 tokens; the plan chosen is within 5 % of
 // the fastest at all but two of those 52 products (8 and 6 %). fp32 activations
 // count three terms. Large tiles fill a CU alone: whole rounds
 // of workgroups. Small ones share it: the longer of one workgroup's latency and
 // the CU's throughput. A split adds its partial tiles' round trip.
 struct TileCost {
-    int tb, rb;
+    int tb, rb, waves;
     bool shared;            // several workgroups per CU
     float step, glu, lin;   // per substep, per workgroup with and without a GLU
     float lstep, lglu, llin;  // the same for a workgroup alone on its CU
 };
 constexpr TileCost kTiles[] = {
-    {16, 4, false, 2.9f, 28.f, 18.f, 0, 0, 0},       {12, 4, false, 2.2f, 26.f, 13.f, 0, 0, 0},
-    {8, 4, false, 1.75f, 16.f, 9.f, 0, 0, 0},        {4, 2, true, 0.62f, 2.0f, 2.f, 0.9f, 5.f, 4.f},
-    {2, 2, true, 0.45f, 1.8f, 1.5f, 0.85f, 4.f, 3.f},
+    {16, 2, 8, false, 2.9f, 28.f, 18.f, 0, 0, 0},       {12, 2, 8, false, 2.2f, 26.f, 13.f, 0, 0, 0},
+    {8, 2, 8, false, 1.75f, 16.f, 9.f, 0, 0, 0},        {4, 2, 4, true, 0.62f, 2.0f, 2.f, 0.9f, 5.f, 4.f},
+    {2, 2, 4, true, 0.45f, 1.8f, 1.5f, 0.85f, 4.f, 3.f},
 };
 
 Plan prefill_plan(int M, int N, int K, int terms, bool glu) {
     const float S = (float)pack_geom(K).S * terms, cus = (float)device_cus();
-    Plan best{4, 2, 1};
+    Plan best{4, 2, 4, 1};
     float least = 0.f;
     for (const TileCost& t : kTiles)
         for (int ks = 1; ks <= 16; ks *= 2) {
-            const int rows = (glu ? 32 : 64) * t.rb;
+            const int rows = (glu ? 8 : 16) * t.waves * t.rb;
             const float tiles = (float)((M + t.tb * 16 - 1) / (t.tb * 16)) * (float)((N + rows - 1) / rows);
             const float s = S / ks, load = tiles * ks / cus;
             if (ks > 1 && (tiles > kSplitCounters || s < 8.f * terms)) break;
             float us = t.shared ? std::max(s * t.lstep + (glu ? t.lglu : t.llin), load * (s * t.step + (glu ? t.glu : t.lin)))
                                 : std::ceil(load) * (s * t.step + (glu ? t.glu : t.lin));
-            if (ks > 1) us += 3.f + 0.164f * ks * t.tb * t.rb;
+            if (ks > 1) us += 3.f + 0.041f * ks * t.tb * t.rb * t.waves;
             if (least == 0.f || us < least) {
                 least = us;
-                best = {t.tb, t.rb, ks};
+                best = {t.tb, t.rb, t.waves, ks};
             }
         }
     return best;
@@ -637,21 +651,22 @@ Plan prefill_plan(int M, int N, int K, int terms, bool glu) {
 template <int TB, int RB, bool GLU>
 hipError_t launch_tile_kernel(const PrefillArgs& a, hipStream_t s) {
     constexpr int kBufs = 2 * prefill_stage<TB>() * TB * kStepBytes;
-    constexpr int kPairs = GLU ? TB * 16 * (32 * RB + 4) * 4 : 0;
+    constexpr int kWaves = prefill_wg<TB, RB>();
+    constexpr int kPairs = GLU ? TB * 16 * (8 * kWaves * RB + 4) * 4 : 0;
     const int lds = kBufs > kPairs ? kBufs : kPairs;
     const void* k = reinterpret_cast<const void*>(&prefill_kernel<TB, RB, GLU>);
     if (lds > 64 * 1024)
         if (hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds); e != hipSuccess) return e;
-    hipLaunchKernelGGL((prefill_kernel<TB, RB, GLU>), dim3(a.tx * a.ty * a.ks), dim3(256), lds, s, a);
+    hipLaunchKernelGGL((prefill_kernel<TB, RB, GLU>), dim3(a.tx * a.ty * a.ks), dim3(64 * kWaves), lds, s, a);
     return hipGetLastError();
 }
 
 template <bool GLU>
 hipError_t launch_plan(const Plan& p, const PrefillArgs& a, hipStream_t s) {
     switch (p.tb * 10 + p.rb) {
-        case 164: return launch_tile_kernel<16, 4, GLU>(a, s);
-        case 124: return launch_tile_kernel<12, 4, GLU>(a, s);
-        case 84: return launch_tile_kernel<8, 4, GLU>(a, s);
+        case 162: return launch_tile_kernel<16, 2, GLU>(a, s);
+        case 122: return launch_tile_kernel<12, 2, GLU>(a, s);
+        case 82: return launch_tile_kernel<8, 2, GLU>(a, s);
         case 42: return launch_tile_kernel<4, 2, GLU>(a, s);
         default: return launch_tile_kernel<2, 2, GLU>(a, s);
     }
@@ -681,7 +696,7 @@ int launch_prefill(const GemvLaunch& L, hipStream_t s, bool* taken) {
     Plan p = prefill_plan(L.M, L.N, L.K, f32 && L.parts == 3 ? 3 : 1, L.glu);
     PrefillArgs a{};
     a.tx = (L.M + p.tb * 16 - 1) / (p.tb * 16);
-    const int rows = (L.glu ? 32 : 64) * p.rb;
+    const int rows = (L.glu ? 8 : 16) * p.waves * p.rb;
     a.ty = (L.N + rows - 1) / rows;
     const int ntile = a.tx * a.ty, tbs = (L.M + 15) / 16;
     Workspace ws{};
@@ -692,7 +707,7 @@ int launch_prefill(const GemvLaunch& L, hipStream_t s, bool* taken) {
     // Scratch: packed activations (unless given), term flags, partial tiles.
     const size_t pack = L.Xp ? 0 : (f32 ? 3 : 1) * xbytes;
     const size_t flag_bytes = f32 ? ((size_t)tbs * pg.nss * 4 + 255) & ~(size_t)255 : 0;
-    const size_t tsz = (size_t)p.tb * p.rb * 1024 * sizeof(float);
+    const size_t tsz = (size_t)p.tb * p.rb * p.waves * 256 * sizeof(float);
     uint8_t* sb = nullptr;
     for (;;) {
         const size_t part = p.ks > 1 ? tsz * p.ks * ntile : 0;
