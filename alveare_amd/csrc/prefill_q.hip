@@ -688,7 +688,9 @@ int launch_prefill(const GemvLaunch& L, hipStream_t s, bool* taken) {
     const uint64_t wbytes = tile_bytes(L.N, L.K);
     const size_t xbytes = packed_bytes(L.M, L.K);
     if (!L.tiled || wbytes >= 0xF0000000ull || xbytes >= 0x7FFFF000ull) return ALV_OK;
-    if (L.Yp && packed_bytes(L.M, L.N) >= 0xFFFFF000ull) return ALV_OK;
+    // (The packed output is the next product's input: blocks past N are padded
+    // to a substep, so it can be the larger of the two.)
+    if (L.Yp && packed_bytes(L.M, L.N) >= 0x7FFFF000ull) return ALV_OK;
     const bool f32 = L.X != nullptr && !L.Xp;
     if (!L.Xp && (f32 ? reinterpret_cast<uintptr_t>(L.X) % 4 != 0 : reinterpret_cast<uintptr_t>(L.Xb) % 16 != 0 || L.ldx % 8 != 0))
         return fail(ALV_ERR_ALIGN, "prefill activations are not aligned for 16-byte loads");
