@@ -26,10 +26,10 @@
 // matrix instructions) at 1.1-1.2 PFLOP/s of the 1.45 that a large bf16 product
 // reaches on this card. Eight waves of two row tiles, two per SIMD, rather than
 // four of four: a wave alone on its SIMD does not overlap its dequantization
-// with its own matrix instructions (512 tokens 194 against 187 us, 3001: 954
-// against 912). FFN 3840 <-> 15360, bf16, us per call, gemm_q.hip before and
-// this kernel: 17 tokens 70 -> 51, 45: 72 -> 60, 128: 111 -> 82, 200: 146 -> 113,
-// 512: 207 -> 187, 3001: 1223 -> 912.
+// with its own matrix instructions (512 tokens 194 against 185 us, 3001: 954
+// against 880). FFN 3840 <-> 15360, bf16, us per call, gemm_q.hip before and
+// this kernel: 17 tokens 70 -> 48, 45: 72 -> 60, 128: 111 -> 77, 200: 146 -> 105,
+// 512: 207 -> 183, 1024: 392 -> 323, 3001: 1224 -> 880.
 //
 // The order of k. A super-step of the tiled layout (512 columns, 16 blocks) is
 // taken in T = 4 substeps of 128: substep t multiplies block T g + t in lane
@@ -608,13 +608,12 @@ struct Plan {
 
 // Tile and K split of a product: the least estimated time over the tiles
 // built. A substep's time and a workgroup's own (prologue, epilogue) are fits,
-// in us, to sweeps of tiles (four-wave ones of 8, 12 and 16 blocks, within 10 %
-// of the eight-wave ones since) and splits over FFNs of 3840 <-> 15360, 1152 <->
-// 6912 and 1056 <-> 14400 at 17 to 3001 tokens; the plan chosen is within 5 % of
-// the fastest at all but two of those 52 products (8 and 6 %). fp32 activations
-// count three terms. Large tiles fill a CU alone: whole rounds
-// of workgroups. Small ones share it: the longer of one workgroup's latency and
-// the CU's throughput. A split adds its partial tiles' round trip.
+// in us, to sweeps of every tile and split over FFNs of 3840 <-> 15360, 1152 <->
+// 6912 and 1056 <-> 14400 at 70 to 3001 tokens; the plan chosen is within 5 % of
+// the fastest at each of those 40 products. fp32 activations count three
+// terms. Large tiles fill a CU alone: whole rounds of workgroups. Small ones
+// share it: the longer of one workgroup's latency and the CU's throughput. A
+// split adds its partial tiles' round trip.
 struct TileCost {
     int tb, rb, waves;
     bool shared;            // several workgroups per CU
@@ -622,9 +621,9 @@ struct TileCost {
     float lstep, lglu, llin;  // the same for a workgroup alone on its CU
 };
 constexpr TileCost kTiles[] = {
-    {16, 2, 8, false, 2.9f, 28.f, 18.f, 0, 0, 0},       {12, 2, 8, false, 2.2f, 26.f, 13.f, 0, 0, 0},
-    {8, 2, 8, false, 1.75f, 16.f, 9.f, 0, 0, 0},        {4, 2, 4, true, 0.62f, 2.0f, 2.f, 0.9f, 5.f, 4.f},
-    {2, 2, 4, true, 0.45f, 1.8f, 1.5f, 0.85f, 4.f, 3.f},
+    {16, 2, 8, false, 2.93f, 20.1f, 15.f, 0, 0, 0},    {12, 2, 8, false, 1.94f, 24.6f, 14.f, 0, 0, 0},
+    {8, 2, 8, false, 1.64f, 15.5f, 7.84f, 0, 0, 0},    {4, 2, 4, true, 0.72f, 2.f, 2.f, 1.17f, 5.f, 4.f},
+    {2, 2, 4, true, 0.54f, 1.8f, 1.29f, 1.05f, 5.36f, 2.91f},
 };
 
 Plan prefill_plan(int M, int N, int K, int terms, bool glu) {
@@ -639,7 +638,7 @@ Plan prefill_plan(int M, int N, int K, int terms, bool glu) {
             if (ks > 1 && (tiles > kSplitCounters || s < 8.f * terms)) break;
             float us = t.shared ? std::max(s * t.lstep + (glu ? t.lglu : t.llin), load * (s * t.step + (glu ? t.glu : t.lin)))
                                 : std::ceil(load) * (s * t.step + (glu ? t.glu : t.lin));
-            if (ks > 1) us += 3.f + 0.041f * ks * t.tb * t.rb * t.waves;
+            if (ks > 1) us += 3.8f + 0.0239f * ks * t.tb * t.rb * t.waves;
             if (least == 0.f || us < least) {
                 least = us;
                 best = {t.tb, t.rb, t.waves, ks};
