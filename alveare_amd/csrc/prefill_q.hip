@@ -181,13 +181,18 @@ struct PrefillArgs {
 // `lds` + 16 lane. Written out because the compiler, which cannot tell the two
 // halves of the LDS buffer apart, would wait for the load before every LDS
 // read; the kernel waits for it (vmcnt) ahead of the barrier that hands the
-// half over.
+// half over. m0 is declared as written, so that the compiler keeps no value of
+// its own there across the statement (it is a reserved register, hence the
+// warning: it is not preserved, as meant).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                  :
                  : "v"(voff), "s"(r), "s"(soff), "s"(lds)
-                 : "memory");
+                 : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 // c += a b on the matrix cores. ACC: written out, with c in accumulation
 // registers, so that the result stays in c's own registers: with some 100 or

@@ -70,3 +70,18 @@ def test_check_catches_the_pattern():
     }
     bad = violations(src)
     assert len(bad) == 2 and all("planted.hip" in b for b in bad), bad
+
+
+def test_m0_writes_are_declared():
+    """An asm statement that writes m0 lists it as clobbered: the compiler may
+    otherwise keep a value of its own there across the statement."""
+    found, bad = 0, []
+    for path in sorted(glob.glob(os.path.join(CSRC, "*.h*")) + glob.glob(os.path.join(ROOT, "measure", "*.hip"))):
+        text = open(path).read()
+        for m in re.finditer(r"\basm\s*(?:volatile)?\s*\((.*?)\);", text, re.S):
+            template = re.match(r'\s*(?:"(?:[^"\\]|\\.)*"\s*)+', m.group(1)).group(0)
+            if re.search(r"\bm0\b", template):
+                found += 1
+                if '"m0"' not in m.group(1)[len(template):]:
+                    bad.append(f"{os.path.basename(path)}:{text.count(chr(10), 0, m.start()) + 1}")
+    assert found and not bad, bad
