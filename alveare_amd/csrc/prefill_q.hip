@@ -200,6 +200,7 @@ __device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, uint32_t vo
 // register files (420 moves per 256 of these) and spilled. It cannot see these writes'
 // latency, so code that reads c otherwise first waits (acc_wait), and a and b
 // are written two instructions or more ahead.
+constexpr int kAccTiles = 24;  // f32x4 accumulators of a lane from which this holds
 template <bool ACC>
 __device__ __forceinline__ void mfma_acc(f32x4& c, bf16x8 a, bf16x8 b) {
     if constexpr (ACC)
@@ -214,7 +215,18 @@ __device__ __forceinline__ void settle(bf16x8 (&b)[RB]) {
     for (int q = 0; q < RB; ++q) asm volatile("" : "+v"(b[q]));
     asm volatile("s_nop 1");
 }
-__device__ __forceinline__ void acc_wait() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+// The accumulators hold the last products. Each is passed through a statement
+// behind the wait: the compiler could otherwise read it ahead of the wait,
+// which touches none of them.
+template <int TB, int RB>
+__device__ __forceinline__ void acc_wait(f32x4 (&acc)[TB][RB]) {
+    if constexpr (TB * RB < kAccTiles) return;  // the compiler's own matrix instructions
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < TB; ++t)
+#pragma unroll
+        for (int q = 0; q < RB; ++q) asm volatile("" : "+a"(acc[t][q]));
+}
 
 // dequant8_mix in 17 steps of one instruction, to be spread between matrix
 // instructions.
@@ -418,7 +430,7 @@ __global__ void __launch_bounds__((64 * prefill_wg<TB, RB>()), (prefill_waves<TB
                     const int f = kk * TB + t;
 #pragma unroll
                     for (int q = 0; q < RB; ++q) {
-                        mfma_acc<(TB * RB >= 24)>(acc[t][q], av[f % R], bv[kk & 1][q]);
+                        mfma_acc<(TB * RB >= kAccTiles)>(acc[t][q], av[f % R], bv[kk & 1][q]);
                         const int slot = (t - G * h) * RB + q;
 #pragma unroll
                         for (int i = 0; i < kDequantSteps; ++i)
@@ -470,7 +482,7 @@ __global__ void __launch_bounds__((64 * prefill_wg<TB, RB>()), (prefill_waves<TB
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
     }
-    acc_wait();
+    acc_wait(acc);
 
     // ---- split K: the last workgroup of the tile adds the partial tiles, in
     // split order (gemm_q.hip's scheme: 16-byte write-through pieces, thread
