@@ -70,8 +70,8 @@ def test_prefill_glu_bits(orc, dev, M, I, act):
     """The epilogue's GLU gives alv_glu's bits (pinned to the reference by
     test_glu_bit_exact) for M x I pairs: gate and up rows that pick one
     activation each. Values over the float32 path's range, its edges and the
-    queue's: |g| from subnormal to 60, zeros, and a token of equal pairs next to
-    a rounding midpoint in every column."""
+    queue's: |g| from subnormal to 60, zeros on either side and whole rows of
+    them, and a token of equal pairs next to a rounding midpoint in every column."""
     import alveare_amd as aa
 
     _say(f"GLU bits M={M} I={I} {act}")
@@ -85,6 +85,11 @@ def test_prefill_glu_bits(orc, dev, M, I, act):
     x[1, :half] = torch.linspace(-12.0, 12.0, half)
     x[2, :half] = -torch.exp2(torch.linspace(-130.0, 5.9, half))
     x[3] = 1.0  # one pair in every column
+    x[4, half:] = 0.0  # zero up beside any gate, zero gate beside any up
+    x[5, :half] = 0.0
+    x[6, :half] = -torch.exp2(torch.linspace(3.0, 127.0, half))  # gates past the exponential's range
+    x[6, half:] = 0.0
+    x[M // 2:M // 2 + 8] = 0.0  # rows of zeros inside a tile
     x = x.to(torch.bfloat16).to(dev)
     y = torch.empty(M, H, dtype=torch.bfloat16, device=dev)
     from alveare_amd import layer
