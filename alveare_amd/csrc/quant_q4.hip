@@ -16,9 +16,12 @@
 // rounding is v_rndne_f32, so the codes match numpy's bit for bit.
 //
 // Eight lanes share a block: lane p holds columns 4p..4p+3 of kQuantRows rows,
-// all loaded (16 bytes each) before the first is needed; a wave covers 8 blocks
-// of a row, so its reads are 1 KiB lines and its writes contiguous. Bound by
-// memory:
+// all loaded (16 bytes each) before the first is needed; a wave covers 8 blocks,
+// of one row where rows are that long, so its reads are 1 KiB lines and its
+// writes contiguous. Blocks follow each other across rows, so that no lane idles
+// at the end of a row (256 columns of one row per wave: 65536 x 64 13.2 us
+// against 7.5, x 544 36.4 against 29.0, 16256 x 4128 68 against 55.5, no
+// difference at multiples of 256). Bound by memory:
 // 3840 x 15360 float32 weights quantized as 4096 x 16384 read and write 278 MB,
 // which a copy at this card's 4.9 TB/s moves in 57 us; they take 58.5. (A block
 // per 8 lanes by a 64-bit division of its number, four 4-byte loads and four
@@ -38,8 +41,7 @@ __device__ __forceinline__ uint32_t bf16_bits_rne(float v) {
     return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
 }
 
-constexpr int kQuantRows = 4;    // rows per wave
-constexpr int kQuantCols = 256;  // columns per wave
+constexpr int kQuantRows = 4;
 
 // max over the 8 lanes of a block (an aligned group, all active): pairs,
 // quads, then the mirrored half row holds the other quad.
@@ -49,65 +51,74 @@ __device__ __forceinline__ uint32_t max8(uint32_t v) {
     return max(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, false));
 }
 
+// kQuantRows rows from r0 on of the block that columns c0 .. c0 + 3 belong to;
+// orow: bytes of an output row.
+__device__ __forceinline__ void quant_rows(const float* W, int n_src, int k_src, int ldw, uint8_t* out, int N,
+                                           size_t orow, int64_t r0, int c0, int part) {
+    float v[kQuantRows][4];
+#pragma unroll
+    for (int t = 0; t < kQuantRows; ++t) {
+        const float* src = W + (size_t)(r0 + t) * ldw + c0;
+        if (r0 + t < n_src && c0 + 3 < k_src) {
+            __builtin_memcpy(v[t], src, sizeof(v[t]));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[t][e] = r0 + t < n_src && c0 + e < k_src ? src[e] : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < kQuantRows; ++t) {
+        if (r0 + t >= N) break;
+        // The largest magnitude by its bits: a NaN's are above infinity's.
+        uint32_t mb = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mb = max(mb, __builtin_bit_cast(uint32_t, v[t][e]) & 0x7FFFFFFFu);
+        mb = max8(mb);
+        float s = mb > 0x7F800000u ? __builtin_nanf("") : __fdiv_rn(__builtin_bit_cast(float, mb), 7.0f);
+        if (s == 0.0f) s = 1.0f;
+        // v / s rounded to an integer: v times the hardware reciprocal is
+        // within 8 * 2^-22 of the quotient (|v / s| < 7.01), so it settles the
+        // integer unless it lies within 2^-18 of a half; then, and for scales
+        // outside the normal range (and NaN), the correctly rounded division.
+        const float rs = __builtin_amdgcn_rcpf(s);
+        float qf[4];
+        bool near = !(s > 1e-30f && s < 1e30f);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float y = v[t][e] * rs;
+            qf[e] = rintf(y);
+            near |= fabsf(y - qf[e]) > 0.5f - 0x1p-18f;
+        }
+        if (near) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) qf[e] = rintf(__fdiv_rn(v[t][e], s));
+        }
+        uint32_t packed = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            int q = qf[e] != qf[e] ? -8 : (int)qf[e];
+            q = q < -8 ? -8 : (q > 7 ? 7 : q);
+            packed |= (uint32_t)(q & 0xF) << (4 * e);
+        }
+        // Even lanes write a dword of two lanes' codes, lane 1 the scale.
+        const uint32_t next = (uint32_t)__builtin_amdgcn_mov_dpp((int)packed, 0xB1, 0xF, 0xF, false);
+        const uint32_t word = part == 1 ? bf16_bits_rne(s) : packed | next << 16;
+        if (part == 1 || !(part & 1))
+            *reinterpret_cast<uint32_t*>(out + (size_t)(r0 + t) * orow + (size_t)(c0 >> 5) * kBlockBytes +
+                                         (part == 1 ? 16 : 2 * part)) = word;
+    }
+}
+
+// Row groups [0, groups) of the rows from row0 on: (group, block) pairs in one
+// sequence, blocks fastest, eight lanes each.
 __global__ void __launch_bounds__(256) quant_kernel(const float* W, int n_src, int k_src, int ldw, uint8_t* out,
-                                                    int N, int K) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, part = lane & 7;
-    const int c0 = blockIdx.x * kQuantCols + lane * 4;
-    if (c0 >= K) return;  // whole blocks: K is a multiple of 32
-    const size_t orow = (size_t)(K / 32) * kBlockBytes;
-    for (int64_t r0 = ((int64_t)blockIdx.y * 4 + wave) * kQuantRows; r0 < N; r0 += (int64_t)gridDim.y * 4 * kQuantRows) {
-        float v[kQuantRows][4];
-#pragma unroll
-        for (int t = 0; t < kQuantRows; ++t) {
-            const float* src = W + (size_t)(r0 + t) * ldw + c0;
-            if (r0 + t < n_src && c0 + 3 < k_src) {
-                __builtin_memcpy(v[t], src, sizeof(v[t]));
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[t][e] = r0 + t < n_src && c0 + e < k_src ? src[e] : 0.0f;
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < kQuantRows; ++t) {
-            if (r0 + t >= N) break;
-            // The largest magnitude by its bits: a NaN's are above infinity's.
-            uint32_t mb = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) mb = max(mb, __builtin_bit_cast(uint32_t, v[t][e]) & 0x7FFFFFFFu);
-            mb = max8(mb);
-            float s = mb > 0x7F800000u ? __builtin_nanf("") : __fdiv_rn(__builtin_bit_cast(float, mb), 7.0f);
-            if (s == 0.0f) s = 1.0f;
-            // v / s rounded to an integer: v times the hardware reciprocal is
-            // within 8 * 2^-22 of the quotient (|v / s| < 7.01), so it settles the
-            // integer unless it lies within 2^-18 of a half; then, and for scales
-            // outside the normal range (and NaN), the correctly rounded division.
-            const float rs = __builtin_amdgcn_rcpf(s);
-            float qf[4];
-            bool near = !(s > 1e-30f && s < 1e30f);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float y = v[t][e] * rs;
-                qf[e] = rintf(y);
-                near |= fabsf(y - qf[e]) > 0.5f - 0x1p-18f;
-            }
-            if (near) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) qf[e] = rintf(__fdiv_rn(v[t][e], s));
-            }
-            uint32_t packed = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                int q = qf[e] != qf[e] ? -8 : (int)qf[e];
-                q = q < -8 ? -8 : (q > 7 ? 7 : q);
-                packed |= (uint32_t)(q & 0xF) << (4 * e);
-            }
-            // Even lanes write a dword of two lanes' codes, lane 1 the scale.
-            const uint32_t next = (uint32_t)__builtin_amdgcn_mov_dpp((int)packed, 0xB1, 0xF, 0xF, false);
-            const uint32_t word = part == 1 ? bf16_bits_rne(s) : packed | next << 16;
-            if (part == 1 || !(part & 1))
-                *reinterpret_cast<uint32_t*>(out + (size_t)(r0 + t) * orow + (size_t)(c0 >> 5) * kBlockBytes +
-                                             (part == 1 ? 16 : 2 * part)) = word;
-        }
+                                                    int N, int K, int64_t row0, uint32_t groups) {
+    const uint32_t nb = (uint32_t)K / 32, total = groups * nb;
+    const int part = threadIdx.x & 7;
+    const size_t orow = (size_t)nb * kBlockBytes;
+    for (uint32_t i = blockIdx.x * 32 + (threadIdx.x >> 3); i < total; i += gridDim.x * 32) {
+        const uint32_t rg = i / nb, b = i - rg * nb;
+        quant_rows(W, n_src, k_src, ldw, out, N, orow, row0 + (int64_t)rg * kQuantRows, (int)(b * 32) + 4 * part, part);
     }
 }
 
@@ -123,10 +134,16 @@ int check_quant(const float* W, int n_src, int k_src, int ldw, const void* out, 
 }
 
 int launch_quant(const float* W, int n_src, int k_src, int ldw, uint8_t* out, int N, int K, hipStream_t s) {
-    const dim3 grid((K + kQuantCols - 1) / kQuantCols,
-                    std::min((N + 4 * kQuantRows - 1) / (4 * kQuantRows), 32768));
-    hipLaunchKernelGGL(quant_kernel, grid, dim3(256), 0, s, W, n_src, k_src, ldw, out, N, K);
-    return hip_check(hipGetLastError(), "quant_kernel launch");
+    // One launch, unless its sequence would pass 2^30 pairs (K / 32 < 2^26 of them per group).
+    const int64_t groups = ((int64_t)N + kQuantRows - 1) / kQuantRows, nb = K / 32, most = (1 << 30) / nb;
+    for (int64_t g0 = 0; g0 < groups; g0 += most) {
+        const int64_t n = std::min(most, groups - g0);
+        const int grid = (int)std::min<int64_t>((n * nb + 31) / 32, 1 << 20);
+        hipLaunchKernelGGL(quant_kernel, dim3(grid), dim3(256), 0, s, W, n_src, k_src, ldw, out, N, K, g0 * kQuantRows,
+                           (uint32_t)n);
+        if (int rc = hip_check(hipGetLastError(), "quant_kernel launch")) return rc;
+    }
+    return ALV_OK;
 }
 
 }  // namespace
