@@ -1,7 +1,9 @@
 // MFMA Q4 GEMM for prefill-sized batches (gfx950) on weights in the combined
 // layout: the path of alv_gemv_q and alv_gemm_q from 33 tokens. Registered
-// weights take prefill_q.hip, and this kernel only where that one's scratch
-// would have to grow during a graph capture or an operand is outside its ranges.
+// weights take prefill_q.hip, and this kernel where it is the faster of the two
+// (lds_tiles_faster: short products, no packing launch), and where that one's
+// scratch would have to grow during a graph capture or an operand is outside
+// its ranges.
 //
 // C[M, N] = X[M, K] * dequant(W)[N, K]^T. A workgroup of 8 waves owns a
 // TM-token x 128-weight-row tile -- TM = 256, or 64 up to 128 tokens (a
@@ -479,10 +481,64 @@ hipError_t launch_gemm_x(const GemmArgs& a, bool xf32, int tm, dim3 grid, hipStr
     return xf32 ? launch_gemm<NT, TILED, true, 256>(a, grid, s) : launch_gemm<NT, TILED, false, 256>(a, grid, s);
 }
 
+// Token tile and K split of a product.
+struct GemmPlan {
+    int TM;
+    dim3 tiles;
+    int ntiles, nsteps, ks;
+};
+
+GemmPlan gemm_plan(int M, int N, int K) {
+    GemmPlan p;
+    // Token tile: 64 for small batches (a quarter of the MFMA and LDS work per
+    // weight tile of the 256-token tile), 256 above small_tile_max_m().
+    p.TM = M <= small_tile_max_m() ? 64 : 256;
+    p.tiles = dim3((M + p.TM - 1) / p.TM, (N + TN - 1) / TN);
+    p.ntiles = (int)(p.tiles.x * p.tiles.y);
+    // Split K while the grid leaves CUs idle and each split keeps enough
+    // steps: 256-token tiles aim at one workgroup per CU (16+ steps each);
+    // 64-token tiles at ALV_GEMM_SMALL_WG_PER_CU workgroups per CU (default
+    // 1; 2-4 measured no faster) with 8+ steps each.
+    p.nsteps = (K + TK - 1) / TK;
+    p.ks = 1;
+    const int wg_target = p.TM == 64 ? small_wg_per_cu() * device_cus() : device_cus();
+    const int min_steps = p.TM == 64 ? 8 : 16;
+    while (p.ntiles * p.ks * 2 <= wg_target && p.nsteps / (p.ks * 2) >= min_steps) p.ks *= 2;
+    return p;
+}
+
 }  // namespace
 
+// `serial`: steps one CU takes after another. The other kernel's packing launch
+// takes 2.5 us and more, and its splits hold twice as many columns at least, so
+// this one wins where little is multiplied (one-term activations: below 512
+// columns; 5.2 against 7.6 us at 3840 x 32 and 48 tokens) and where its grid
+// and split meet the CUs exactly (8192 x 3840, 64 tokens: 18.5 against 20.0 us,
+// 18.9 against 22.4 with weights from memory; 1536 x 1152, 4096 tokens: 27.1
+// against 31.3). Three terms are three passes here, so little is left of it.
+// Lines drawn over 22000 random products of 64-262144 rows, 32-16384 columns
+// and 17-4096 tokens: always packing was over 6 % slower than this kernel at
+// 2600 of them (up to 1.7 times), with the rule at 130 (up to 1.24).
+bool lds_tiles_faster(int M, int N, int K, bool three) {
+    const GemmPlan p = gemm_plan(M, N, K);
+    const int cus = device_cus(), serial = (p.ntiles * p.ks + cus - 1) / cus * ((p.nsteps + p.ks - 1) / p.ks);
+    const bool round = p.ntiles <= cus, small = p.TM == 64;
+    if (three) {
+        if (small) return K <= 64 || (K < 512 && round && p.ntiles > cus / 2);
+        return p.ntiles > cus / 4 && (K <= 64 || (K <= 384 && round));
+    }
+    if (K < 512) return small || K <= 128 || p.ntiles > cus / 6;
+    if (small)
+        return (K > 2048 && serial >= 10 && serial < 16) || (K <= 10240 && N <= 2048 && p.ks >= 4) ||
+               (round && p.ntiles > 5 * cus / 8 && serial < 16);
+    return round && serial <= 18 && p.ntiles > (M > 2048 ? cus / 2 : 5 * cus / 8);
+}
+
 int launch_gemm_tiled(const GemvLaunch& L, hipStream_t s) {
-    if (L.tiled && !L.glu) {
+    bool xf32 = L.Xb == nullptr;
+    const uint64_t xbytes = ((uint64_t)(L.M - 1) * L.ldx + L.K) * (xf32 ? 4 : 2);
+    const bool xfits = xbytes < 0x7FFFFF00ull;
+    if (L.tiled && !L.glu && !(xfits && lds_tiles_faster(L.M, L.N, L.K, xf32 && L.parts == 3))) {
         bool taken = false;
         if (int rc = launch_prefill(L, s, &taken)) return rc;
         if (taken) return launch_zero_rows(L, s);
@@ -492,29 +548,17 @@ int launch_gemm_tiled(const GemvLaunch& L, hipStream_t s) {
     // 3.75 GiB, activations below 2 GiB.
     if (wbytes >= 0xF0000000ull) return fail(ALV_ERR_RANGE, "weight matrix of %llu bytes exceeds the 3.75 GiB prefill range", (unsigned long long)wbytes);
     if (L.parts != 1 && L.parts != 3) return fail(ALV_ERR_ARG, "parts must be 1 or 3");
-    bool xf32 = L.Xb == nullptr;
     const void* x = xf32 ? static_cast<const void*>(L.X) : static_cast<const void*>(L.Xb);
     // 16-byte activation loads: 4-byte aligned rows for fp32; for bf16 (the FFN's
     // own activation buffer) 16-byte aligned rows.
     if (xf32 ? reinterpret_cast<uintptr_t>(x) % 4 != 0 : reinterpret_cast<uintptr_t>(x) % 16 != 0 || L.ldx % 8 != 0)
         return fail(ALV_ERR_ALIGN, "prefill activations are not aligned for 16-byte loads");
-    uint64_t xbytes = ((uint64_t)(L.M - 1) * L.ldx + L.K) * (xf32 ? 4 : 2);
-    if (xbytes >= 0x7FFFFF00ull) return fail(ALV_ERR_RANGE, "activations of %llu bytes exceed the 2 GiB buffer range", (unsigned long long)xbytes);
+    if (!xfits) return fail(ALV_ERR_RANGE, "activations of %llu bytes exceed the 2 GiB buffer range", (unsigned long long)xbytes);
     const int NT = L.glu ? 2 : 1;
-    // Token tile: 64 for small batches (a quarter of the MFMA and LDS work per
-    // weight tile of the 256-token tile), 256 above small_tile_max_m().
-    const int TM = L.M <= small_tile_max_m() ? 64 : 256;
-    const dim3 tiles((L.M + TM - 1) / TM, (L.N + TN - 1) / TN);
-    const int ntiles = (int)(tiles.x * tiles.y);
-    // Split K while the grid leaves CUs idle and each split keeps enough
-    // steps: 256-token tiles aim at one workgroup per CU (16+ steps each);
-    // 64-token tiles at ALV_GEMM_SMALL_WG_PER_CU workgroups per CU (default
-    // 1; 2-4 measured no faster) with 8+ steps each.
-    const int nsteps = (L.K + TK - 1) / TK;
-    int ks = 1;
-    const int wg_target = TM == 64 ? small_wg_per_cu() * device_cus() : device_cus();
-    const int min_steps = TM == 64 ? 8 : 16;
-    while (ntiles * ks * 2 <= wg_target && nsteps / (ks * 2) >= min_steps) ks *= 2;
+    const GemmPlan plan = gemm_plan(L.M, L.N, L.K);
+    const dim3 tiles = plan.tiles;
+    const int TM = plan.TM, ntiles = plan.ntiles;
+    int ks = plan.ks;
     // Split-K arrival counters: the stream's dedicated counter words (zero
     // between launches, shared with the streaming kernel's split K), never
     // the scratch below, whose bytes hold other launches' flags and terms.

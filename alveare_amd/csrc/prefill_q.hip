@@ -1,6 +1,7 @@
 // Prefill products on registered (tiled) weights for gfx950: the path of
-// alv_gemv, alv_gemv_bf16, alv_ffn_fused and alv_ffn_fused_bf16 from 17 (bf16
-// activations) or 33 (fp32) tokens.
+// alv_gemv, alv_gemv_bf16 (but where gemm_q.hip's lds_tiles_faster says
+// otherwise), alv_ffn_fused and alv_ffn_fused_bf16 from 17 (bf16 activations) or
+// 33 (fp32) tokens.
 //
 // C[M, N] = X[M, K] * dequant(W)[N, K]^T in two launches:
 //   1. pack_x_kernel lays the activations out once in MFMA operand order
@@ -773,3 +774,16 @@ int launch_prefill(const GemvLaunch& L, hipStream_t s, bool* taken) {
 }
 
 }  // namespace alv
+
+extern "C" int alv_prefill_plan(int M, int N, int K, int fp32, int glu, int* tokens, int* splits) {
+    using namespace alv;
+    if (!tokens || !splits) return fail(ALV_ERR_ARG, "null pointer");
+    if (M < 1 || N < 1 || K < 32 || K % 32) return fail(ALV_ERR_ARG, "bad shape M=%d N=%d K=%d", M, N, K);
+    *tokens = 0;
+    *splits = 0;
+    if (!glu && lds_tiles_faster(M, N, K, fp32 != 0)) return ALV_OK;
+    const Plan p = prefill_plan(M, N, K, fp32 ? 3 : 1, glu != 0);
+    *tokens = 16 * p.tb;
+    *splits = p.ks;
+    return ALV_OK;
+}

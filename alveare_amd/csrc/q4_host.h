@@ -141,6 +141,10 @@ constexpr int kGemvMaxM = 16;
 // GemvLaunch (glu pairs W0/W1 into the activation).
 int launch_gemm_tiled(const GemvLaunch& L, hipStream_t s);
 
+// Whether the kernel of gemm_q.hip takes a product on registered weights in less
+// time than launch_prefill (three: fp32 activations in three terms).
+bool lds_tiles_faster(int M, int N, int K, bool three);
+
 // The same product with the weights dequantized into operand registers and the
 // activations packed in operand order (prefill_q.hip); registered weights
 // only. *taken false (and nothing enqueued): the shape is outside its ranges,

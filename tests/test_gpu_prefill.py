@@ -24,22 +24,50 @@ def _weight(orc, dev, N, K, seed):
     return aa.Q4Weight(W, N, K), aa.dequant_q4(W, N, K).double()
 
 
-# tile (16-token blocks x 16-row blocks per wave) and split the plan picks: 2x2;
-# 2x2, two blocks; 4x2 split twice; 2x2 split 8 times (30 whole super-steps);
-# 4x2 split 8 times; 8x4, ragged rows; 12x4; 16x4, ragged tokens and rows.
-SHAPES = [(17, 333, 480), (31, 1000, 32), (600, 2000, 3872), (70, 512, 15360), (600, 544, 15360), (193, 30001, 544),
-          (300, 30720, 1024), (490, 30000, 1056)]
+def _plan(M, N, K, fp32=False, glu=False):
+    """(tokens per workgroup, K splits) of the prefill kernel, (0, 0) for the
+    LDS tile kernel of csrc/gemm_q.hip."""
+    import ctypes
+
+    import alveare_amd as aa
+
+    t, k = ctypes.c_int(), ctypes.c_int()
+    aa._lib.check(aa.lib().alv_prefill_plan(M, N, K, int(fp32), int(glu), ctypes.byref(t), ctypes.byref(k)), "plan")
+    return t.value, k.value
+
+
+# M, N, K and the plan of a 256-CU card: every tile, unsplit and at splits the
+# plan takes, token and row remainders, whole (1984) and partial super-steps; then
+# the LDS tile kernel on registered weights, 64- and 256-token tiles.
+PRODUCTS = {
+    "bf16": [(18, 69, 576, 32, 1), (130, 333, 480, 32, 1), (21, 67, 1984, 32, 2), (138, 67, 4000, 32, 4),
+             (18, 69, 16064, 32, 8), (19, 69, 16288, 32, 16), (98, 20247, 544, 64, 1), (33, 23714, 1984, 64, 2),
+             (2849, 131, 4000, 64, 4), (33, 6369, 8128, 64, 8), (290, 19501, 544, 128, 1), (68, 31169, 3424, 128, 2),
+             (71, 16299, 5920, 128, 4), (265, 29911, 544, 192, 1), (132, 28098, 3648, 192, 2), (129, 15296, 7456, 192, 4),
+             (775, 13825, 544, 256, 1),
+             (17, 333, 480, 0, 0), (31, 1000, 32, 0, 0), (64, 8192, 3840, 0, 0), (1000, 1111, 96, 0, 0),
+             (3000, 1536, 1152, 0, 0),
+             (600, 2000, 3872, 64, 2), (70, 512, 15360, 0, 0), (600, 544, 15360, 64, 8),
+             (193, 30001, 544, 0, 0), (300, 30720, 1024, 192, 1), (490, 30000, 1056, 256, 1)],
+    "fp32": [(34, 96, 1984, 32, 2), (37, 69, 5152, 32, 4), (36, 96, 16288, 32, 16), (70, 28608, 96, 64, 1),
+             (34, 10048, 4160, 64, 4), (67, 21920, 2336, 128, 2), (69, 8128, 8160, 128, 8), (276, 22304, 544, 192, 1),
+             (131, 7008, 8352, 192, 8), (390, 22112, 576, 256, 1), (206, 25152, 6048, 256, 2),
+             (33, 333, 64, 0, 0), (700, 9000, 160, 0, 0),
+             (600, 2000, 3872, 64, 2), (70, 512, 15360, 32, 8), (600, 544, 15360, 64, 8),
+             (193, 30001, 544, 128, 1), (300, 30720, 1024, 192, 1), (490, 30000, 1056, 256, 1)],
+}
 
 
 # (fp32 activations take the streaming kernel below 33 tokens)
-@pytest.mark.parametrize("M,N,K,dtype", [(*s, d) for s in SHAPES for d in ("bf16", "fp32") if d == "bf16" or s[0] > 32])
-def test_prefill_products(orc, dev, M, N, K, dtype):
+@pytest.mark.parametrize("M,N,K,tokens,splits,dtype", [(*s, d) for d, shapes in PRODUCTS.items() for s in shapes])
+def test_prefill_products(orc, dev, M, N, K, tokens, splits, dtype):
     """Within the float32 bound of the float64 product: K + 8 roundings of 2^-24
     over sum |x w| (three terms: 3 K + 8), a bf16 result half a bf16 ulp more
     (2^-8 of the value: eight significant bits)."""
     from alveare_amd import layer
 
     _say(f"product M={M} N={N} K={K} {dtype}")
+    assert _plan(M, N, K, dtype == "fp32") == (tokens, splits)
     w, w64 = _weight(orc, dev, N, K, M + N)
     x = torch.from_numpy(orc.synth_normal(M * K, M + K)).to(dev).view(M, K)
     x = x.to(torch.bfloat16) if dtype == "bf16" else x
