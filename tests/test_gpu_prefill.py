@@ -92,9 +92,16 @@ def _picker(I, H, cols):
     return W.reshape(I, -1)
 
 
-@pytest.mark.parametrize("act", ["gelu", "silu"])
-@pytest.mark.parametrize("M,I", [(480, 15360), (330, 2080), (17, 2080)])
-def test_prefill_glu_bits(orc, dev, M, I, act):
+# M, I, H (the K of gate/up) and its plan: every tile, unsplit and split.
+GLU = [(480, 15360, 1056, 256, 1), (17, 2080, 1056, 32, 1), (330, 2080, 1056, 32, 1), (17, 96, 1984, 32, 2),
+       (26, 64, 4000, 32, 4), (65, 13152, 544, 64, 1), (33, 10176, 2176, 64, 2), (33, 5440, 4032, 64, 4),
+       (33, 3008, 8608, 64, 8), (76, 31840, 864, 128, 1), (67, 16256, 5312, 128, 2), (66, 8160, 9568, 128, 4),
+       (137, 31552, 736, 192, 1), (129, 13472, 5248, 192, 2), (142, 7872, 8416, 192, 4), (446, 6272, 15136, 256, 2)]
+
+
+@pytest.mark.parametrize("M,I,H,tokens,splits,act", [(*s, a) for i, s in enumerate(GLU)
+                                                     for a in (("gelu", "silu") if i < 3 else ("gelu",))])
+def test_prefill_glu_bits(orc, dev, M, I, H, tokens, splits, act):
     """The epilogue's GLU gives alv_glu's bits (pinned to the reference by
     test_glu_bit_exact) for M x I pairs: gate and up rows that pick one
     activation each. Values over the float32 path's range, its edges and the
@@ -102,8 +109,9 @@ def test_prefill_glu_bits(orc, dev, M, I, act):
     them, and a token of equal pairs next to a rounding midpoint in every column."""
     import alveare_amd as aa
 
-    _say(f"GLU bits M={M} I={I} {act}")
-    H, half = 1056, 528
+    _say(f"GLU bits M={M} I={I} H={H} {act}")
+    assert _plan(M, I, H, glu=True) == (tokens, splits)
+    half = H // 2
     rows = np.arange(I)
     ffn = aa.pack_ffn_fused_weights(_picker(I, H, rows % half), _picker(I, H, half + rows // half),
                                     orc.synth_q4(H, I, 5), H, I, activation=act, device=dev)
@@ -160,6 +168,50 @@ def test_prefill_scratch_holds_no_old_values(orc, dev):
     assert (y.double() - ref).abs().max() <= 2.0 ** -8 * ref.abs().max()
     big.close()
     ffn.close()
+
+
+def test_prefill_ffn_capture_fallback(orc, dev):
+    """An FFN captured on a stream whose scratch holds its activation but not its
+    packed input runs the LDS tile kernels, the activation row-major: alv_glu's
+    bits, and the down product's bound, at every replay."""
+    import alveare_amd as aa
+    from alveare_amd import layer
+
+    _say("FFN capture without packing scratch")
+    H, I, M = 4096, 512, 200  # 1.6 MB packed, 0.2 MB of activation; scratch grows by whole MiB
+    half, rows = H // 2, np.arange(I)
+    Wd = orc.synth_q4(H, I, 5)
+    ffn = aa.pack_ffn_fused_weights(_picker(I, H, rows % half), _picker(I, H, half + rows), Wd, H, I, device=dev)
+    small = aa.pack_ffn_fused_weights(orc.synth_q4(512, 64, 1), orc.synth_q4(512, 64, 2), orc.synth_q4(64, 512, 3), 64,
+                                      512, device=dev)
+    x = torch.from_numpy(orc.synth_normal(M * H, 7)).to(dev).view(M, H).to(torch.bfloat16)
+    xs = torch.ones(40, 64, dtype=torch.bfloat16, device=dev)
+    w64 = aa.dequant_q4(torch.from_numpy(Wd).to(dev), H, I).double()
+    gg, uu = (x[:, c].float().contiguous() for c in (torch.from_numpy(rows % half).to(dev), torch.from_numpy(half + rows).to(dev)))
+    want = torch.empty_like(gg)
+    y = torch.empty(M * H, dtype=torch.bfloat16, device=dev)
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream(device=dev)
+    with torch.cuda.stream(s):
+        aa._lib.check(aa.lib().alv_glu(gg.data_ptr(), uu.data_ptr(), want.data_ptr(), gg.numel(), 0, s.cuda_stream), "alv_glu")
+        layer.ffn_fused_bf16(small, xs, M=40)
+        s.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            layer.ffn_fused_bf16(ffn, x, y, M)
+        ref = want.double() @ w64.T
+        bound = (I + 8) * 2.0 ** -24 * (want.double().abs() @ w64.abs().T) * 1.01 + ref.abs() * 2.0 ** -8 + 1e-30
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            got = ffn.last_activation(M)
+            s.synchronize()
+            assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+            assert ((y.view(M, H).double() - ref).abs() <= bound).all()
+            layer.ffn_fused_bf16(small, xs, M=40)
+            s.synchronize()
+    ffn.close()
+    small.close()
 
 
 def test_prefill_capture(orc, dev):

@@ -5,7 +5,7 @@ import os
 
 import pytest
 
-from test_gpu_prefill import PRODUCTS
+from test_gpu_prefill import GLU, PRODUCTS
 
 
 @pytest.fixture(scope="module")
@@ -25,15 +25,17 @@ def plan():
 
 
 def test_cases_run_the_tiles_they_name(plan):
-    """The GPU tests' products still have the plans listed beside them, and
-    together cover every tile built, unsplit and split."""
+    """The GPU tests' products and FFNs still have the plans listed beside them,
+    and together cover every tile built, unsplit and split."""
     for dtype, shapes in PRODUCTS.items():
         for M, N, K, *want in shapes:
             assert plan(M, N, K, dtype == "fp32") == tuple(want), (M, N, K, dtype)
+    for M, I, H, *want in GLU:
+        assert plan(M, I, H, glu=True) == tuple(want), (M, I, H)
     tiles = {32, 64, 128, 192, 256}
-    cases = [tuple(s[3:]) for shapes in PRODUCTS.values() for s in shapes]
-    assert tiles <= {t for t, k in cases if k == 1}
-    assert tiles <= {t for t, k in cases if k > 1}
+    for cases in ([tuple(s[3:]) for shapes in PRODUCTS.values() for s in shapes], [s[3:] for s in GLU]):
+        assert tiles <= {t for t, k in cases if k == 1}
+        assert tiles <= {t for t, k in cases if k > 1}
 
 
 @pytest.mark.parametrize("M,N,K,fp32,lds", [
