@@ -238,19 +238,26 @@ def test_qkv_attention_fused_bit_identical(dev, sliding, pos):
     assert np.array_equal(bf_np(vc_a), bf_np(vc_b))
 
 
+def _wide(rows, heads, window=0):
+    """launch_attention's rule for sixteen 512-wide heads per workgroup, one kv head."""
+    return heads % 16 == 0 and -(-min(window or rows, rows) // 64) * (heads // 16) >= 64
+
+
 @pytest.mark.parametrize("pos,window,heads,half,v_off", [(0, 0, 16, 256, -1), (1, 0, 16, 64, 0), (62, 0, 32, 0, -1),
-                                                          (63, 0, 16, 256, 0), (64, 0, 16, 37, 0), (500, 100, 16, 256, 0),
-                                                          (2047, 0, 16, 256, -1), (2047, 0, 32, 256, 0)])
+                                                          (63, 0, 16, 256, 0), (64, 0, 16, 37, 0), (500, 4096, 16, 256, 0),
+                                                          (2047, 0, 16, 256, -1), (1000, 0, 32, 256, 0),
+                                                          (1023, 2048, 32, 128, -1)])
 def test_attention_wide_bit_identical(dev, pos, window, heads, half, v_off):
-    """From a 4096-position cache on, 16 q heads of 512 per workgroup on the
-    matrix cores give, bit for bit, what the two-head workgroups of a
-    2048-position cache give on the same rows: attention output, rotated q and
-    both cache rows, through both entry points (chunk edges, one position, a
-    window, two workgroups per chunk, RoPE of all, some and no values)."""
+    """From 64 workgroups on, 16 q heads of 512 per workgroup on the matrix cores
+    give, bit for bit, what the two-head workgroups of a shorter cache give on
+    the same rows: attention output, rotated q and both cache rows, through both
+    entry points (chunk edges, one position, two workgroups per chunk, RoPE of
+    all, some and no values)."""
     from alveare_amd import layer
 
     _say(f"wide attention pos={pos} window={window} heads={heads} half={half}")
-    D, S, wide = 512, 2048, 4096
+    D, S, wide = 512, 2048 if heads == 16 else 1024, 4096 if heads == 16 else 2048
+    assert not _wide(S, heads, window) and _wide(wide, heads, window)
     rng = np.random.default_rng(pos + heads + half)
     qkv = bf_dev(rnd_bf16(rng, (heads + 2) * D, 1.0), dev)
     kc0, vc0 = rnd_bf16(rng, (1, S, D), 0.2), rnd_bf16(rng, (1, S, D), 1.0)
@@ -277,6 +284,78 @@ def test_attention_wide_bit_identical(dev, pos, window, heads, half, v_off):
     assert not np.isnan(got[0][0]).any()
     for narrow, w in zip(*got):
         assert np.array_equal(narrow, w)
+
+
+@pytest.mark.parametrize("heads,pos", [(16, 6000), (32, 4160)])
+def test_attention_wide_window(dev, heads, pos):
+    """A window that starts past row 0 (spans this long are wide in any cache)
+    gives the bits of the same rows at the head of a cache of their own, and the
+    float64 attention within the bound of the chunks' float32 sums: 2^-8 of the
+    value for the bf16 result, (64 + 512 + 8) 2^-24 relative in the weights and
+    sums of the largest magnitudes."""
+    from alveare_amd import layer
+
+    D, W, S = 512, 4096, 8192
+    _say(f"wide attention, window of {W} at {pos}, {heads} heads")
+    assert _wide(S, heads, W) and _wide(W, heads) and pos >= W
+    rng = np.random.default_rng(pos)
+    q = bf_dev(rnd_bf16(rng, heads * D, 0.06), dev)
+    kc, vc = (bf_dev(rnd_bf16(rng, (1, S, D), 1.0), dev).view(1, S, D) for _ in range(2))
+    lo = pos + 1 - W
+    kc[:, :lo] = float("nan")  # rows outside the window are not read into any sum
+    vc[:, :lo] = float("nan")
+    kc[:, pos + 1:] = float("nan")
+    vc[:, pos + 1:] = float("nan")
+    out = layer.attention(q, kc, vc, torch.tensor([pos], dtype=torch.int32, device=dev), heads=heads, window=W)
+    ks, vs = (c[:, lo:pos + 1].contiguous() for c in (kc, vc))
+    head = layer.attention(q, ks, vs, torch.tensor([W - 1], dtype=torch.int32, device=dev), heads=heads)
+    torch.cuda.synchronize()
+    assert np.array_equal(bf_np(out), bf_np(head))
+    s = q.double().view(heads, D) @ ks[0].double().T
+    p = torch.softmax(s, dim=-1)
+    ref = p @ vs[0].double()
+    eps = (64 + 512 + 8) * 2.0 ** -24
+    mag = (q.double().abs().view(heads, D) @ ks[0].double().abs().T).max().item()  # a score's error times this
+    bound = ref.abs() * 2.0 ** -8 + 2 * (1 + mag) * eps * (p @ vs[0].double().abs())
+    assert ((out.double().view(heads, D) - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("data", ["subnormal", "underflow", "huge", "inf_k", "inf_v", "nan_v"])
+def test_attention_wide_extreme_values(dev, data):
+    """The matrix cores' chains give the bits of the two-head workgroups' fmaf
+    where products, sums and weights are subnormal, weights underflow to zero,
+    sums reach 1e38, and where a row holds infinities or NaN."""
+    from alveare_amd import layer
+
+    heads, D, pos = 16, 512, 1990
+    _say(f"wide attention on {data} values")
+    rng = np.random.default_rng(len(data))
+    q, k, v = (torch.from_numpy(rng.standard_normal(n).astype(np.float32)) for n in (heads * D, 2048 * D, 2048 * D))
+    scale = 1.0
+    if data == "subnormal":  # products near 1e-40, their sums scaled up into the softmax; V below 2^-126
+        q, k, v, scale = q * 1e-20, k * 1e-20, v * 2.0 ** -127, 1e38
+    elif data == "underflow":  # scores spread over hundreds: most weights are subnormal or zero
+        q, v = q * 4, v * 2.0 ** -100
+    elif data == "huge":
+        q, k, v, scale = q * 1e17, k * 1e17, v * 1e35, 1e-35
+    elif data == "inf_k":
+        k[1990 * D + 5] = float("inf")  # the chunk's last row
+    else:
+        v[1990 * D + 5] = float("inf" if data == "inf_v" else "nan")
+        v[700 * D + 9] = float("-inf")
+    q, k, v = (t.to(torch.bfloat16).to(dev) for t in (q, k, v))
+    pos_dev = torch.tensor([pos], dtype=torch.int32, device=dev)
+    got = []
+    for rows in (2048, 4096):
+        kc, vc = (torch.zeros((1, rows, D), dtype=torch.bfloat16, device=dev) for _ in range(2))
+        kc[0, :2048], vc[0, :2048] = k.view(2048, D), v.view(2048, D)
+        got.append(parity.bf16_bits(layer.attention(q, kc, vc, pos_dev, heads=heads, scale=scale)))
+    assert not _wide(2048, heads) and _wide(4096, heads)
+    nan = [(g & 0x7FFF) > 0x7F80 for g in got]  # a NaN's bits are not fixed
+    assert np.array_equal(nan[0], nan[1])
+    assert np.array_equal(np.where(nan[0], 0, got[0]), np.where(nan[1], 0, got[1]))
+    if data == "subnormal":
+        assert ((got[0] & 0x7FFF) < 0x0080).all() and (got[0] & 0x7FFF).any()
 
 
 # ---- residual steps (model.py:775-788; model.cpp:409-420) ---------------------------
