@@ -2,8 +2,10 @@
 
 The compiler tracks no hazard of an inline-asm matrix instruction and does not
 see its latency. Checked for every instance built: no operand is written by a
-vector instruction within two wait states before the instruction, and an
-accumulator leaves it through the statements after acc_wait alone."""
+vector instruction within two wait states before the instruction, an
+accumulator leaves it through the statements after acc_wait alone, and a counted
+wait for the loads into LDS leaves no more in flight than was asked for after
+them."""
 import os
 import re
 import subprocess
@@ -77,6 +79,33 @@ def hazards(body):
     return checked, bad
 
 
+def open_waits(body):
+    """Counted (nonzero) hand-written load waits of one kernel's assembly that a
+    load into LDS could still be pending behind: fewer vector memory
+    instructions than the count, or a label, stand between the last such load
+    and the wait. Returns (waits checked, those found)."""
+    checked, bad = 0, []
+    since = None  # vector memory instructions since the last load into LDS
+    inline = False
+    for line in body.splitlines():
+        if ";#ASM" in line:
+            inline = "#ASMSTART" in line
+            continue
+        text = line.split(";")[0].strip()
+        if re.match(r"[.\w$]+:$", text):
+            since = None
+        elif re.match(r"buffer_load\w* .*\blds$", text):
+            since = 0
+        elif re.match(r"(buffer|global|flat|scratch)_(load|store|atomic)", text) and since is not None:
+            since += 1
+        m = re.match(r"s_waitcnt vmcnt\((\d+)\)$", text)
+        if inline and m and int(m.group(1)):
+            checked += 1
+            if since is None or since < int(m.group(1)):
+                bad.append(f"{text} after {since}")
+    return checked, bad
+
+
 def early_reads(ir):
     """Uses of an inline-asm matrix instruction's result, itself or through
     phis, by anything but another inline-asm statement, in one IR function."""
@@ -109,6 +138,15 @@ def test_matrix_operands_settle(compiled):
     assert total > 0
 
 
+def test_lds_loads_land_before_the_barrier(compiled):
+    total = 0
+    for name, body in re.findall(r"^(\w+prefill_kernel\w+):(.*?)\.end_amdhsa_kernel", compiled[0], re.S | re.M):
+        checked, bad = open_waits(body)
+        total += checked
+        assert not bad, f"{name}: {bad[:3]}"
+    assert total >= 20  # at least one per stage of a super-step
+
+
 def test_accumulators_read_after_the_wait(compiled):
     found = 0
     for m in re.finditer(r"^define [^\n]*@(\w*prefill_kernel\w*)\(.*?^}", compiled[1], re.S | re.M):
@@ -124,6 +162,11 @@ def test_checks_find_planted_faults():
     assert hazards(asm) == (1, ["v_mfma_f32_16x16x32_bf16 a[0:3], v[4:7], v[8:11], a[0:3]"])
     assert hazards(asm.replace("s_nop 0", "s_nop 1")) == (1, [])
     assert len(hazards(asm.replace("s_nop 0", "s_nop 1\n.LBB0_1:"))[1]) == 1
+    load = "\tbuffer_load_dwordx4 v1, s[0:3], s4 offen lds\n\tbuffer_load_dwordx4 v[2:5], v1, s[0:3], 0 offen\n"
+    wait = "\t;;#ASMSTART\n\ts_waitcnt vmcnt(%d)\n\t;;#ASMEND\n"
+    assert open_waits(load + wait % 1) == (1, [])
+    assert open_waits(load + wait % 2) == (1, ["s_waitcnt vmcnt(2) after 1"])
+    assert len(open_waits(load + ".LBB0_1:\n" + wait % 1)[1]) == 1
     ir = ('  %1 = call <4 x float> asm sideeffect "v_mfma $0", "=a"()\n  %2 = phi <4 x float> [ %1, %3 ]\n'
           "  %4 = extractelement <4 x float> %2, i64 0\n")
     assert early_reads(ir)[1] == ["extractelement <4 x float> %2, i64 0"]
