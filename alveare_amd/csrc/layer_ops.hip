@@ -541,8 +541,8 @@ __global__ void __launch_bounds__(kAttnThreads) attn_partial_kernel(AttnArgs a) 
 // Sixteen q heads per workgroup at D = 512, for long spans, on the matrix
 // cores: K and V read once instead of once per two heads, and every result bit
 // that of the partial kernel. v_mfma_f32_16x16x4_f32 adds its four products in
-// order, each by one fused multiply-add (checked against fmaf on random data
-// down to subnormals, test_attention_wide_bit_identical), so a chain of them
+// order, each by one fused multiply-add (test_attention_wide_bit_identical, and
+// test_attention_wide_extreme_values from subnormals to NaN), so a chain of them
 // over k is the chain of fmaf it replaces. A = the 16 heads' q values (weights),
 // B = 16 positions' K values (16 columns' V values), widened from bf16.
 //   * Scores: wave w takes quarter w % 4 of the columns (the partial kernel's

@@ -20,9 +20,12 @@
 // Activations go from memory straight into LDS (buffer_load ... lds), whole
 // operand fragments of 1 KiB, and are read without bank conflicts.
 //
-// What bounds it: up to 128 tokens the dequantization (68 VALU clocks per 16 x
-// 32 weights a wave, as many as 4.25 matrix instructions) and the launches'
-// latency; above, LDS reads (every wave reads all of the workgroup's
+// What bounds it: up to 128 tokens waiting, for the L2 (a substep's activations
+// are asked for one substep ahead) and for issue. Gate/up of 3840 <-> 15360 at 45
+// tokens, 33.8 us: the matrix cores busy 21 % of the time and the vector ALUs
+// 36 % (68 clocks of dequantization per 16 x 32 weights a wave, 6.4 us of it),
+// a wave's time 38 % at s_waitcnt or a barrier and 27 % at an instruction that is
+// ready. Above, LDS reads (every wave reads all of the workgroup's
 // activations, 512 KiB per 256 x 256 x 128 substep: 4096 clocks, as many as its
 // matrix instructions) at 1.1-1.2 PFLOP/s of the 1.45 that a large bf16 product
 // reaches on this card. Eight waves of two row tiles, two per SIMD, rather than
@@ -266,19 +269,19 @@ constexpr int prefill_stage() {
 
 // Waves per workgroup: eight, two per SIMD, where a CU's LDS and registers hold
 // one such workgroup; four, several workgroups per CU, for small tiles.
-template <int TB, int RB>
+template <int TB>
 constexpr int prefill_wg() {
     return TB >= 8 ? 8 : 4;
 }
 
-template <int TB, int RB>
+template <int TB>
 constexpr int prefill_waves() {  // waves per SIMD the register budget is set for
     return TB >= 8 ? 2 : 3;
 }
 
 template <int TB, int RB, bool GLU>
-__global__ void __launch_bounds__((64 * prefill_wg<TB, RB>()), (prefill_waves<TB, RB>())) prefill_kernel(PrefillArgs a) {
-    constexpr int NWV = prefill_wg<TB, RB>(), NT = 64 * NWV;
+__global__ void __launch_bounds__((64 * prefill_wg<TB>()), (prefill_waves<TB>())) prefill_kernel(PrefillArgs a) {
+    constexpr int NWV = prefill_wg<TB>(), NT = 64 * NWV;
     constexpr int RBM = GLU ? RB / 2 : RB;  // row tiles of one matrix per wave
     constexpr int PS = prefill_stage<TB>();      // substeps per stage: an LDS buffer, a barrier
     constexpr int BUF = PS * TB * kStepBytes;    // one LDS buffer
@@ -383,7 +386,7 @@ __global__ void __launch_bounds__((64 * prefill_wg<TB, RB>()), (prefill_waves<TB
     // other's latest loads), and the next substep's first octet follows. A
     // group is one row tile's dequantization between the matrix instructions
     // of G fragments.
-    constexpr int G = TB / RB, R = RB >= 4 ? 4 : NWV == 8 ? 6 : 8 < 4 * TB ? 8 : 4 * TB;  // R: operand reads ahead
+    constexpr int G = TB / RB, R = NWV == 8 ? 6 : 8;  // R: operand reads ahead
     constexpr int XL = 4 * TB / NWV;  // fragments a wave loads per substep
     constexpr int LK = PS, LG = (PS * XL + LK * RB - 1) / (LK * RB);  // activation loads: over LK octets, per group
     static_assert(TB % RB == 0, "whole fragments per group");
@@ -627,9 +630,12 @@ struct Plan {
 // Tile and K split of a product: the least estimated time over the tiles
 // built. A substep's time and a workgroup's own (prologue, epilogue) are fits,
 // in us, to sweeps of every tile and split over FFNs of 3840 <-> 15360, 1152 <->
-// 6912 and 1056 <-> 14400 at 70 to 3001 tokens; the plan chosen is within 5 % of
-// the fastest at each of those 40 products. fp32 activations count three
-// terms. Large tiles fill a CU alone: whole rounds of workgroups. Small ones
+// 6912 and 1056 <-> 14400 at 70 to 3001 tokens. At 17 to 512 tokens an FFN with
+// the plan's tiles takes at most 4 % more than with the fastest pair of tiles and
+// splits at 3840 <-> 15360, 12 % at 1152 <-> 6912, 2048 <-> 8192 and 1056 <->
+// 14400 (the fit's sizes begin at 70 tokens); 2100 one-term projections at 17 to
+// 4096 tokens 2.4 % in the mean, one in twenty over 11 %. fp32 activations count
+// three terms. Large tiles fill a CU alone: whole rounds of workgroups. Small ones
 // share it: the longer of one workgroup's latency and the CU's throughput. A
 // split adds its partial tiles' round trip.
 struct TileCost {
@@ -668,7 +674,7 @@ Plan prefill_plan(int M, int N, int K, int terms, bool glu) {
 template <int TB, int RB, bool GLU>
 hipError_t launch_tile_kernel(const PrefillArgs& a, hipStream_t s) {
     constexpr int kBufs = 2 * prefill_stage<TB>() * TB * kStepBytes;
-    constexpr int kWaves = prefill_wg<TB, RB>();
+    constexpr int kWaves = prefill_wg<TB>();
     constexpr int kPairs = GLU ? TB * 16 * (8 * kWaves * RB + 4) * 4 : 0;
     const int lds = kBufs > kPairs ? kBufs : kPairs;
     const void* k = reinterpret_cast<const void*>(&prefill_kernel<TB, RB, GLU>);
@@ -775,14 +781,15 @@ int launch_prefill(const GemvLaunch& L, hipStream_t s, bool* taken) {
 
 }  // namespace alv
 
-extern "C" int alv_prefill_plan(int M, int N, int K, int fp32, int glu, int* tokens, int* splits) {
+extern "C" int alv_prefill_plan(int M, int N, int K, int fp32, int ffn, int* tokens, int* splits) {
     using namespace alv;
     if (!tokens || !splits) return fail(ALV_ERR_ARG, "null pointer");
     if (M < 1 || N < 1 || K < 32 || K % 32) return fail(ALV_ERR_ARG, "bad shape M=%d N=%d K=%d", M, N, K);
     *tokens = 0;
     *splits = 0;
-    if (!glu && lds_tiles_faster(M, N, K, fp32 != 0)) return ALV_OK;
-    const Plan p = prefill_plan(M, N, K, fp32 ? 3 : 1, glu != 0);
+    if (ffn < 0 || ffn > 2) return fail(ALV_ERR_ARG, "ffn must be 0, 1 or 2 (got %d)", ffn);
+    if (!ffn && lds_tiles_faster(M, N, K, fp32 != 0)) return ALV_OK;
+    const Plan p = prefill_plan(M, N, K, fp32 && ffn < 2 ? 3 : 1, ffn == 1);
     *tokens = 16 * p.tb;
     *splits = p.ks;
     return ALV_OK;

@@ -303,7 +303,7 @@ __device__ __forceinline__ bool glu_fast(float g, float u, int act, float* out) 
 }
 
 // The GELU fast path in fewer instructions (prefill_q.hip: a tile's epilogue
-// evaluates 128 values per lane): z's factor, -2 and log2(e) are one constant c
+// evaluates 64 values per lane): z's factor, -2 and log2(e) are one constant c
 // and the hardware's exp2 and reciprocal take the place of expf and the
 // division. t = c inner: c and the product round by 1.5 * 2^-24 of |t| <= 31.8,
 // 33.1 * 2^-24 through 2^t; exp2 and the reciprocal 1 ulp each (2 * 2^-24),

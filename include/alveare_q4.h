@@ -131,12 +131,13 @@ int alv_gemv_bf16(alv_weight_t w, const uint16_t* X, uint16_t* Y, int M, int ldx
 
 /*
  * The route of a prefill-sized product on registered weights at its executed
- * shape (fp32: activations in three terms; glu: an FFN's gate/up): *tokens per
+ * shape (fp32: activations in three terms; ffn: 0 a projection, 1 an FFN's
+ * gate/up, 2 its down product of bf16 activations): *tokens per
  * workgroup of the prefill kernel and its K *splits, or 0 and 0 where the LDS
  * tile kernel takes it. No device work, no reference counterpart: it lets a
  * test tell which kernel it runs.
  */
-int alv_prefill_plan(int M, int N, int K, int fp32, int glu, int* tokens, int* splits);
+int alv_prefill_plan(int M, int N, int K, int fp32, int ffn, int* tokens, int* splits);
 
 /* Free a handle from alv_weight_register (NULL is a no-op). Synchronises the
  * device before freeing. */

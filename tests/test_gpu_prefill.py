@@ -24,7 +24,7 @@ def _weight(orc, dev, N, K, seed):
     return aa.Q4Weight(W, N, K), aa.dequant_q4(W, N, K).double()
 
 
-def _plan(M, N, K, fp32=False, glu=False):
+def _plan(M, N, K, fp32=False, ffn=0):
     """(tokens per workgroup, K splits) of the prefill kernel, (0, 0) for the
     LDS tile kernel of csrc/gemm_q.hip."""
     import ctypes
@@ -32,7 +32,7 @@ def _plan(M, N, K, fp32=False, glu=False):
     import alveare_amd as aa
 
     t, k = ctypes.c_int(), ctypes.c_int()
-    aa._lib.check(aa.lib().alv_prefill_plan(M, N, K, int(fp32), int(glu), ctypes.byref(t), ctypes.byref(k)), "plan")
+    aa._lib.check(aa.lib().alv_prefill_plan(M, N, K, int(fp32), ffn, ctypes.byref(t), ctypes.byref(k)), "plan")
     return t.value, k.value
 
 
@@ -110,7 +110,7 @@ def test_prefill_glu_bits(orc, dev, M, I, H, tokens, splits, act):
     import alveare_amd as aa
 
     _say(f"GLU bits M={M} I={I} H={H} {act}")
-    assert _plan(M, I, H, glu=True) == (tokens, splits)
+    assert _plan(M, I, H, ffn=1) == (tokens, splits)
     half = H // 2
     rows = np.arange(I)
     ffn = aa.pack_ffn_fused_weights(_picker(I, H, rows % half), _picker(I, H, half + rows // half),

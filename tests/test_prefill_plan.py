@@ -16,9 +16,9 @@ def plan():
         build.build()
     L = _lib.lib()
 
-    def f(M, N, K, fp32=False, glu=False):
+    def f(M, N, K, fp32=False, ffn=0):
         t, k = ctypes.c_int(), ctypes.c_int()
-        assert L.alv_prefill_plan(M, N, K, int(fp32), int(glu), ctypes.byref(t), ctypes.byref(k)) == 0
+        assert L.alv_prefill_plan(M, N, K, int(fp32), ffn, ctypes.byref(t), ctypes.byref(k)) == 0
         return t.value, k.value
 
     return f
@@ -31,7 +31,7 @@ def test_cases_run_the_tiles_they_name(plan):
         for M, N, K, *want in shapes:
             assert plan(M, N, K, dtype == "fp32") == tuple(want), (M, N, K, dtype)
     for M, I, H, *want in GLU:
-        assert plan(M, I, H, glu=True) == tuple(want), (M, I, H)
+        assert plan(M, I, H, ffn=1) == tuple(want), (M, I, H)
     tiles = {32, 64, 128, 192, 256}
     for cases in ([tuple(s[3:]) for shapes in PRODUCTS.values() for s in shapes], [s[3:] for s in GLU]):
         assert tiles <= {t for t, k in cases if k == 1}
@@ -48,7 +48,8 @@ def test_short_products_keep_the_lds_kernel(plan, M, N, K, fp32, lds):
     """Both sides of the rule's lines at sizes where the packing launch was
     measured slower, and where it was measured faster."""
     assert (plan(M, N, K, bool(fp32)) == (0, 0)) == lds
-    assert plan(M, N, K, bool(fp32), True) != (0, 0)  # an FFN's gate/up always packs
+    assert plan(M, N, K, bool(fp32), 1) != (0, 0)  # an FFN's products always pack
+    assert plan(M, N, K, False, 2) != (0, 0)
 
 
 def test_plan_refuses_what_no_product_has(plan):
@@ -57,4 +58,5 @@ def test_plan_refuses_what_no_product_has(plan):
     L, t = _lib.lib(), ctypes.c_int()
     for M, N, K in ((0, 1, 32), (1, 0, 32), (1, 1, 0), (1, 1, 48)):
         assert L.alv_prefill_plan(M, N, K, 0, 0, ctypes.byref(t), ctypes.byref(t)) == _lib.ALV_ERR_ARG
+    assert L.alv_prefill_plan(1, 1, 32, 0, 3, ctypes.byref(t), ctypes.byref(t)) == _lib.ALV_ERR_ARG
     assert L.alv_prefill_plan(1, 1, 32, 0, 0, None, ctypes.byref(t)) == _lib.ALV_ERR_ARG
