@@ -52,7 +52,6 @@ namespace alv {
 
 namespace {
 
-constexpr int kQueue = 1024;  // values of a tile the GLU's float32 path may leave
 constexpr int kFragBytes = 1024;
 constexpr int kStepBytes = 4 * kFragBytes;  // 16 tokens x one substep
 
@@ -278,6 +277,12 @@ template <int TB>
 constexpr int prefill_waves() {  // waves per SIMD the register budget is set for
     return TB >= 8 ? 2 : 3;
 }
+
+// The GLU epilogue's LDS row of (gate, up) pairs, and its queue of values the
+// float32 path leaves: less than one round of the nt threads kept, and all of
+// two octets per thread.
+constexpr int glu_stride(int rows) { return rows + 4; }
+constexpr int glu_queue(int nt) { return nt + 16 * nt; }
 
 template <int TB, int RB, bool GLU>
 __global__ void __launch_bounds__((64 * prefill_wg<TB>()), (prefill_waves<TB>())) prefill_kernel(PrefillArgs a) {
@@ -529,14 +534,22 @@ __global__ void __launch_bounds__((64 * prefill_wg<TB>()), (prefill_waves<TB>())
     if constexpr (GLU) {
         // bf16 (gate, up) pairs of the tile into LDS, then whole octets of the
         // activation to memory in operand order (sixteen tokens' octet is 256
-        // contiguous bytes). Values the float32 path cannot settle (about one
-        // in 500) are queued and evaluated together: one by one where they
-        // occur, nearly every octet's wave would run the float64 path.
-        constexpr int NR = 16 * NWV * RBM, LS = NR + 4;  // rows, LDS row stride in pairs
+        // contiguous bytes). Values the float32 path cannot settle (one in 500
+        // of ordinary gates, one in 20 where gates spread over +-10) are queued
+        // and evaluated together, a round of the workgroup's threads at a time:
+        // one by one where they occur, nearly every octet's wave would run the
+        // float64 path. (512 tokens of 3840 <-> 15360, gates 3.4 wide: 183 us,
+        // as with gates 1 wide; 213 with gemm_q.hip, and 239 when more misses
+        // than a queue for the tile held sent all of it to the float64 path.)
+        constexpr int NR = 16 * NWV * RBM, LS = glu_stride(NR);  // rows, LDS row stride in pairs
+        constexpr int OCTETS = TB * 16 * (NR / 8), BATCH = 2 * NT;  // BATCH: between two looks at the queue
+        static_assert(TB * 16 * LS <= 65536, "16-bit queue entries");
         uint32_t* tile = reinterpret_cast<uint32_t*>(smem);
-        __shared__ int queued, queue[kQueue];
-        bool over = false;
-        if (tid == 0) queued = 0;
+        uint16_t* queue = reinterpret_cast<uint16_t*>(tile + TB * 16 * LS);  // glu_queue(NT) entries
+        constexpr int BATCHES = (OCTETS + BATCH - 1) / BATCH;
+        __shared__ int queued[BATCHES];  // by each batch: stable once a barrier has ended it
+        int waiting = 0;                 // by the batches before, not yet evaluated
+        if (tid < BATCHES) queued[tid] = 0;
 #pragma unroll
         for (int t = 0; t < TB; ++t)
 #pragma unroll
@@ -551,51 +564,55 @@ __global__ void __launch_bounds__((64 * prefill_wg<TB>()), (prefill_waves<TB>())
         const PackGeom po = pack_geom(a.N);
         const int n0 = ty * NR;
 #pragma unroll 1
-        for (int c = tid; c < TB * 16 * (NR / 8); c += NT) {
-            const int i = c & 15, o = (c >> 4) % (NR / 8), t = (c >> 4) / (NR / 8);
-            const int m = m0 + 16 * t + i, n = n0 + 8 * o;
-            if (m0 + 16 * t >= a.M || n >= a.N) continue;
-            const u32x4* src = reinterpret_cast<const u32x4*>(tile + (16 * t + i) * LS + 8 * o);
-            const u32x4 p0 = src[0], p1 = src[1];
-            const uint32_t pk[8] = {p0[0], p0[1], p0[2], p0[3], p1[0], p1[1], p1[2], p1[3]};
-            bf16x8 y;
-            uint32_t miss = 0;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                float v = 0.0f;
-                if (a.act != ALV_ACT_GELU_TANH)
-                    v = glu_exact(lo_half(pk[e]), hi_half(pk[e]), a.act);
-                else if (!gelu_quick(lo_half(pk[e]), hi_half(pk[e]), &v))
-                    miss |= 1u << e;
-                y[e] = (__bf16)v;
-            }
-            if (m >= a.M) miss = 0;
-            uint16_t* dst = reinterpret_cast<uint16_t*>(a.Yp + pack_offset(po, m, n >> 3));
-            *reinterpret_cast<u32x4*>(dst) = m < a.M ? __builtin_bit_cast(u32x4, y) : u32x4{0, 0, 0, 0};
-            while (miss) {
-                const int e = __builtin_ctz(miss);
-                miss &= miss - 1;
-                const int at = atomicAdd(&queued, 1);
-                if (at < kQueue)
-                    queue[at] = ((16 * t + i) * LS + 8 * o + e);
-                else
-                    over = true;
-            }
-        }
-        // What the float32 path left: an entry per thread, once the octets
-        // around it are in memory. (More than the queue holds: every value of
-        // the tile again.)
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        const bool all = __syncthreads_or(over);
-        const int nq = all ? TB * 16 * NR : queued;
+        for (int b = 0; b < BATCHES; ++b) {
 #pragma unroll 1
-        for (int c = tid; c < nq; c += NT) {
-            const int at = all ? c / NR * LS + c % NR : queue[c];
-            const int mt = at / LS, nt = at - mt * LS;
-            if (m0 + mt >= a.M || n0 + nt >= a.N) continue;
-            const uint32_t w = tile[at];
-            reinterpret_cast<uint16_t*>(a.Yp + pack_offset(po, m0 + mt, (n0 + nt) >> 3))[(n0 + nt) & 7] =
-                __builtin_bit_cast(uint16_t, (__bf16)glu_exact(lo_half(w), hi_half(w), a.act));
+            for (int c = b * BATCH + tid; c < min(b * BATCH + BATCH, OCTETS); c += NT) {
+                const int i = c & 15, o = (c >> 4) % (NR / 8), t = (c >> 4) / (NR / 8);
+                const int m = m0 + 16 * t + i, n = n0 + 8 * o;
+                if (m0 + 16 * t >= a.M || n >= a.N) continue;
+                const u32x4* src = reinterpret_cast<const u32x4*>(tile + (16 * t + i) * LS + 8 * o);
+                const u32x4 p0 = src[0], p1 = src[1];
+                const uint32_t pk[8] = {p0[0], p0[1], p0[2], p0[3], p1[0], p1[1], p1[2], p1[3]};
+                bf16x8 y;
+                uint32_t miss = 0;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    float v = 0.0f;
+                    if (a.act != ALV_ACT_GELU_TANH)
+                        v = glu_exact(lo_half(pk[e]), hi_half(pk[e]), a.act);
+                    else if (!gelu_quick(lo_half(pk[e]), hi_half(pk[e]), &v))
+                        miss |= 1u << e;
+                    y[e] = (__bf16)v;
+                }
+                if (m >= a.M) miss = 0;
+                uint16_t* dst = reinterpret_cast<uint16_t*>(a.Yp + pack_offset(po, m, n >> 3));
+                *reinterpret_cast<u32x4*>(dst) = m < a.M ? __builtin_bit_cast(u32x4, y) : u32x4{0, 0, 0, 0};
+                while (miss) {
+                    const int e = __builtin_ctz(miss);
+                    miss &= miss - 1;
+                    queue[waiting + atomicAdd(&queued[b], 1)] = (uint16_t)((16 * t + i) * LS + 8 * o + e);
+                }
+            }
+            // A whole round waits (or no more will come): an entry per thread,
+            // once the octets around it are in memory.
+            const bool end = b == BATCHES - 1;
+            if (end) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            waiting += queued[b];
+            if (waiting < NT && !end) continue;
+            if (!end) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+            }
+#pragma unroll 1
+            for (int c = tid; c < waiting; c += NT) {
+                const int at = queue[c], mt = at / LS, nt = at - mt * LS;
+                const uint32_t w = tile[at];
+                reinterpret_cast<uint16_t*>(a.Yp + pack_offset(po, m0 + mt, (n0 + nt) >> 3))[(n0 + nt) & 7] =
+                    __builtin_bit_cast(uint16_t, (__bf16)glu_exact(lo_half(w), hi_half(w), a.act));
+            }
+            waiting = 0;
+            if (!end) __syncthreads();
         }
         // Blocks past the last, up to a whole substep, are zeros: their weights
         // are, and what the buffer held before may not be finite.
@@ -675,8 +692,9 @@ template <int TB, int RB, bool GLU>
 hipError_t launch_tile_kernel(const PrefillArgs& a, hipStream_t s) {
     constexpr int kBufs = 2 * prefill_stage<TB>() * TB * kStepBytes;
     constexpr int kWaves = prefill_wg<TB>();
-    constexpr int kPairs = GLU ? TB * 16 * (8 * kWaves * RB + 4) * 4 : 0;
-    const int lds = kBufs > kPairs ? kBufs : kPairs;
+    constexpr int kPairs = GLU ? TB * 16 * glu_stride(8 * kWaves * RB) * 4 + glu_queue(64 * kWaves) * 2 : 0;
+    constexpr int lds = kBufs > kPairs ? kBufs : kPairs;
+    static_assert(lds + 64 <= 160 * 1024, "LDS of a CU");
     const void* k = reinterpret_cast<const void*>(&prefill_kernel<TB, RB, GLU>);
     if (lds > 64 * 1024)
         if (hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds); e != hipSuccess) return e;

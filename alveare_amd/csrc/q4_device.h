@@ -311,17 +311,20 @@ __device__ __forceinline__ bool glu_fast(float g, float u, int act, float* out) 
 // 45 fp32 ulps of v at most, against the 64 of the midpoint test. A zero factor
 // beside a finite one settles too: both ways give the zero of sign(g) sign(u)
 // (padding tokens are rows of such pairs; 2000 tokens, half of them zeros,
-// through 1152 <-> 6912: 138 us, 264 with their pairs on the float64 path).
+// through 1152 <-> 6912: 138 us, 264 with their pairs on the float64 path). So
+// does z < -22 (t > 64), where 1 + tanh(z) = 2e^-44 is 0 in float64 and the
+// result the zero of sign(g) sign(u).
 __device__ __forceinline__ bool gelu_quick(float g, float u, float* out) {
 #pragma clang fp contract(off)
     const float g3 = (g * g) * g;
     const float inner = g + 0.044715f * g3;
     const float t = -2.3022081986f * inner;  // -2 sqrt(2 / pi) log2(e)
-    const float v = (g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t))) * u;
+    const float f = t > 64.0f ? 0.0f : __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t));
+    const float v = (g * f) * u;
     const uint32_t b = __builtin_bit_cast(uint32_t, v);
     const uint32_t mag = b & 0x7FFFFFFFu;
     *out = v;
-    if (v == 0.0f && (g == 0.0f || u == 0.0f)) return true;
+    if (v == 0.0f && (g == 0.0f || u == 0.0f || f == 0.0f)) return true;
     return t <= 31.7f && mag >= 0x04000000u && mag < 0x7E800000u && (b & 0xFFFFu) - 0x7FC0u > 0x80u;
 }
 

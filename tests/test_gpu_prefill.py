@@ -125,6 +125,7 @@ def test_prefill_glu_bits(orc, dev, M, I, H, tokens, splits, act):
     x[5, :half] = 0.0
     x[6, :half] = -torch.exp2(torch.linspace(3.0, 127.0, half))  # gates past the exponential's range
     x[6, half:] = 0.0
+    x[7, :half] = -torch.linspace(4.0, 40.0, half)  # 1 + tanh from ordinary to zero in float64
     x[M // 2:M // 2 + 8] = 0.0  # rows of zeros inside a tile
     x = x.to(torch.bfloat16).to(dev)
     y = torch.empty(M, H, dtype=torch.bfloat16, device=dev)
@@ -144,6 +145,37 @@ def test_prefill_glu_bits(orc, dev, M, I, H, tokens, splits, act):
     ref = got.double() @ w64.T
     bound = (I + 8) * 2.0 ** -24 * (got.double().abs() @ w64.abs().T) + ref.abs() * 2.0 ** -8 + 1e-30
     assert ((y.double() - ref).abs() <= 1.01 * bound).all()
+    ffn.close()
+
+
+@pytest.mark.parametrize("M,I,H,tokens,splits", [GLU[0], GLU[1], GLU[5], GLU[9], GLU[12]])
+@pytest.mark.parametrize("share", [0.01, 0.05, 0.3, 1.0])
+def test_prefill_glu_queue(orc, dev, M, I, H, tokens, splits, share):
+    """Gates between -7.6 and -5.7, which only the float64 path settles, in a
+    hundredth to all of the values: the queue is drained between batches, at its
+    limit, and at the tile's end, with the bits of alv_glu."""
+    import alveare_amd as aa
+    from alveare_amd import layer
+
+    _say(f"GLU queue M={M} I={I} H={H}, {share} of the gates")
+    assert _plan(M, I, H, ffn=1) == (tokens, splits)
+    half, rows = H // 2, np.arange(I)
+    ffn = aa.pack_ffn_fused_weights(_picker(I, H, rows % half), _picker(I, H, half + rows // half),
+                                    orc.synth_q4(H, I, 5), H, I, device=dev)
+    g = torch.Generator().manual_seed(M + I)
+    x = torch.randn(M, H, generator=g)
+    band = -5.7 - 1.9 * torch.rand(M, half, generator=g)
+    x[:, :half] = torch.where(torch.rand(M, half, generator=g) < share, band, x[:, :half])
+    x = x.to(torch.bfloat16).to(dev)
+    layer.ffn_fused_bf16(ffn, x, M=M)
+    got = ffn.last_activation(M)
+    cols = torch.from_numpy(rows).to(dev)
+    gg, uu = x.float()[:, cols % half].contiguous(), x.float()[:, half + cols // half].contiguous()
+    want = torch.empty_like(gg)
+    aa._lib.check(aa.lib().alv_glu(gg.data_ptr(), uu.data_ptr(), want.data_ptr(), gg.numel(), 0,
+                                   torch.cuda.current_stream().cuda_stream), "alv_glu")
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
     ffn.close()
 
 
