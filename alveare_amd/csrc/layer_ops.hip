@@ -856,9 +856,12 @@ __global__ void __launch_bounds__(kWideThreads) attn_wide_kernel(AttnArgs a) {
 // by all of them, kMergeStage chunks at a time (48 KiB); one thread per column
 // (and one for the denominator) then adds in chunk order. 188 chunks of 16
 // heads of 512: 6 us; with one thread evaluating the factors and 32 workgroups
-// of 256 columns, 8 loads in flight each, 20.
+// of 256 columns, 8 loads in flight each, 20. Up to kMergeWave chunks (a window
+// of 1024) one wave does all of it from registers, without barriers: both
+// launches at position 63 of a 1024 window, 8 kv heads of 256, 8.4 us against 9.0.
 constexpr int kMergeThreads = 512;
 constexpr int kMergeStage = 192;
+constexpr int kMergeWave = 16;  // chunks one wave merges from its registers
 
 __global__ void __launch_bounds__(kMergeThreads) attn_merge_kernel(AttnArgs a) {
     constexpr int NW = kMergeThreads / 64, NB = 8;  // NB: loads per batch
@@ -875,6 +878,29 @@ __global__ void __launch_bounds__(kMergeThreads) attn_merge_kernel(AttnArgs a) {
     const int nch = attn_span(a, pos).nch;
     const float* base = a.part + ((size_t)kvh * a.nchunk * g + hl) * gstride;  // chunk q at + q * g * gstride
     const float* col = base + blockIdx.y * 64 + lane;
+    if (nch <= kMergeWave) {
+        if (wave) return;
+        const float* ml = base + (size_t)min(lane, nch - 1) * g * gstride + D;  // lane q: chunk q's
+        const float mq = ml[0], lq = ml[1];
+        float v[kMergeWave];
+#pragma unroll
+        for (int q = 0; q < kMergeWave; ++q) v[q] = col[(size_t)min(q, nch - 1) * g * gstride];
+        float m = fmaxf(-__builtin_inff(), mq);
+        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+        const float f = expf(mq - m);
+        auto of = [](float x, int q) __attribute__((always_inline)) {
+            return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), q));
+        };
+        float O = 0.0f, L = 0.0f;
+#pragma unroll
+        for (int q = 0; q < kMergeWave; ++q)
+            if (q < nch) {
+                O = fmaf(v[q], of(f, q), O);
+                L = fmaf(of(lq, q), of(f, q), L);
+            }
+        a.out[(size_t)hq * D + blockIdx.y * 64 + lane] = bf16_rne_bits(__fdiv_rn(O, L));
+        return;
+    }
     // Chunks [q0, q0 + kMergeStage) of the 64 columns, every load of a wave in
     // flight at once (a chunk past the last reads it again).
     auto stage = [&](int q0) __attribute__((always_inline)) {
@@ -1160,7 +1186,10 @@ int launch_attention(AttnArgs& a, bool fused, hipStream_t s) {
     // workgroup against sixteen: 2048-position cache 14.8 against 16.4 at
     // position 1500; 4096: 15.1 / 16.5 at 1500, 25.8 / 18.7 at 4000; 12288:
     // 16.5 / 16.5 at 1500, 64.7 / 23.4 at 12000; 32768: 20.4 / 16.4 at 1500,
-    // 166 / 47 at 32000.
+    // 166 / 47 at 32000. (The position is known on the device only, so short
+    // spans of a long cache pay for it: 15.9 at position 63 of 4096, 14.1 with
+    // workgroups of two heads; over all positions of a 4096, 8192 and 12288 cache
+    // it takes 0.78, 0.54 and 0.41 of their time.)
     const bool wide = D == kWideD && g % kWideHeads == 0 && (long)nchunk * kv_heads * (g / kWideHeads) >= kWideMinGrid;
     if (wide) hg = kWideHeads;
     a.g = g;

@@ -252,7 +252,7 @@ def test_attention_wide_bit_identical(dev, pos, window, heads, half, v_off):
     give, bit for bit, what the two-head workgroups of a shorter cache give on
     the same rows: attention output, rotated q and both cache rows, through both
     entry points (chunk edges, one position, two workgroups per chunk, RoPE of
-    all, some and no values)."""
+    all, some and no values, each norm left out)."""
     from alveare_amd import layer
 
     _say(f"wide attention pos={pos} window={window} heads={heads} half={half}")
@@ -263,6 +263,8 @@ def test_attention_wide_bit_identical(dev, pos, window, heads, half, v_off):
     kc0, vc0 = rnd_bf16(rng, (1, S, D), 0.2), rnd_bf16(rng, (1, S, D), 1.0)
     qw, kw = rng.uniform(0.1, 0.3, D).astype(np.float32), rng.uniform(0.1, 0.3, D).astype(np.float32)
     pos_dev = torch.tensor([pos], dtype=torch.int32, device=dev)
+    norms = {1: (False, True, True), 63: (True, False, True), 64: (True, True, False), 2047: (False,) * 3}
+    norm_q, norm_k, norm_v = norms.get(pos, (True,) * 3)
     got = []
     for rows in (S, wide):
         kc = torch.zeros((1, rows, D), dtype=torch.bfloat16, device=dev)
@@ -275,8 +277,8 @@ def test_attention_wide_bit_identical(dev, pos, window, heads, half, v_off):
         rope = dict(rope=table, rope_stride=512, cos_off=0, sin_off=256, half=half) if half else {}
         q = torch.empty(heads * D, dtype=torch.bfloat16, device=dev)
         out = layer.qkv_attention(qkv, pos_dev, kc, vc, heads=heads, kv_heads=1, D=D, k_off=heads * D,
-                                  v_off=(heads + 1) * D if v_off >= 0 else -1, q_w=qw, k_w=kw, q_out=q, window=window,
-                                  **rope)
+                                  v_off=(heads + 1) * D if v_off >= 0 else -1, q_w=qw, k_w=kw, norm_q=norm_q,
+                                  norm_k=norm_k, norm_v=norm_v, q_out=q, window=window, **rope)
         again = layer.attention(q, kc, vc, pos_dev, heads=heads, window=window)
         torch.cuda.synchronize()
         assert np.array_equal(bf_np(out), bf_np(again))
@@ -318,6 +320,28 @@ def test_attention_wide_window(dev, heads, pos):
     mag = (q.double().abs().view(heads, D) @ ks[0].double().abs().T).max().item()  # a score's error times this
     bound = ref.abs() * 2.0 ** -8 + 2 * (1 + mag) * eps * (p @ vs[0].double().abs())
     assert ((out.double().view(heads, D) - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("heads,kv,D", [(4, 1, 64), (16, 8, 256), (16, 1, 512)])
+@pytest.mark.parametrize("pos", [0, 63, 64, 1022, 1023, 1024, 1025, 2047])
+def test_attention_merge_edges(dev, heads, kv, D, pos):
+    """Either side of the 16 chunks that one wave merges: the float64 attention
+    within half a bf16 ulp (2^-8 of the value) and the chunks' float32 sums."""
+    from alveare_amd import layer
+
+    _say(f"merge at position {pos}, {heads} heads on {kv} of {D}")
+    rng = np.random.default_rng(pos + D)
+    q = bf_dev(rnd_bf16(rng, heads * D, D ** -0.5), dev)
+    kc, vc = (bf_dev(rnd_bf16(rng, (kv, 2048, D), 1.0), dev).view(kv, 2048, D) for _ in range(2))
+    out = layer.attention(q, kc, vc, torch.tensor([pos], dtype=torch.int32, device=dev), heads=heads)
+    ks, vs = (c[:, :pos + 1].double() for c in (kc, vc))
+    q64 = q.double().view(kv, heads // kv, D)
+    p = torch.softmax(q64 @ ks.transpose(1, 2).contiguous(), dim=-1)
+    ref = p @ vs
+    eps = (64 + D + 40) * 2.0 ** -24  # a chunk's sums, a score's, the merge's
+    mag = (q64.abs() @ ks.abs().transpose(1, 2).contiguous()).max().item()
+    bound = ref.abs() * 2.0 ** -8 + 2 * (1 + mag) * eps * (p @ vs.abs())
+    assert ((out.double().view(ref.shape) - ref).abs() <= bound).all()
 
 
 @pytest.mark.parametrize("data", ["subnormal", "underflow", "huge", "inf_k", "inf_v", "nan_v"])
