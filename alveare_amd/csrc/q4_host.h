@@ -163,11 +163,11 @@ int launch_zero_rows(const GemvLaunch& L, hipStream_t s);
 // environment variable ALV_TILED_MIN_M, read at each call, overrides both (a
 // tuning knob; the benchmark times both kernels at small M with it).
 // Measured on the 12B-class FFN (3840 <-> 15360), 16 distinct layers, µs
-// per call: streaming 53-56 at 16 tokens and 82-84 at 17 (two launches);
-// tiled with 64-token tiles 78-80 for any M up to 64 with bf16-valued
-// activations and 133-138 with fp32 ones; so from 17 tokens the tiled kernel
-// wins for bf16 (78 against 82), and from 33 for fp32 (streaming 106 at 32,
-// 148 at 40, against 135-138).
+// per call: streaming 49 at 16 bf16-valued tokens and 80 at 17 (two launches),
+// the prefill kernel 53 for any M up to 32; so from 17 tokens it wins for bf16.
+// The fp32 line dates from gemm_q.hip's kernel (133-138 up to 64 tokens, against
+// streaming 106 at 32 and 148 at 40); the prefill kernel takes 82-84 up to 32,
+// less than streaming from 20 tokens (87) on.
 constexpr int kTiledMinMBf16 = 17;
 constexpr int kTiledMinMF32 = 33;
 int tiled_min_m(bool fp32_x);

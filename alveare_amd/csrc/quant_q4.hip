@@ -23,7 +23,7 @@
 // against 7.5, x 544 36.4 against 29.0, 16256 x 4128 68 against 55.5, no
 // difference at multiples of 256). Bound by memory:
 // 3840 x 15360 float32 weights quantized as 4096 x 16384 read and write 278 MB,
-// which a copy at this card's 4.9 TB/s moves in 57 us; they take 58.5. (A block
+// which a copy at this card's 4.9 TB/s moves in 57 us; they take 54. (A block
 // per 8 lanes by a 64-bit division of its number, four 4-byte loads and four
 // IEEE divisions per lane took 82.)
 #include <algorithm>

@@ -27,10 +27,10 @@ import statistics
 import sys
 from collections import defaultdict
 
-Q4_KERNELS = ("q4_gemv1_kernel", "q4_gemv1_step_kernel", "gemm_q4_kernel", "tile_kernel", "rmsnorm_kernel", "qkv_post_kernel",
-              "attn_partial_kernel", "attn_merge_kernel", "add_norm_kernel", "embed_kernel", "head_kernel",
-              "head_fold_kernel", "quant_kernel", "split_x_kernel", "split_fix_kernel", "q4_ffn1_kernel",
-              "ffn1_sum_kernel", "ffn1_vdown_kernel")
+Q4_KERNELS = ("q4_gemv1_kernel", "q4_gemv1_step_kernel", "gemm_q4_kernel", "prefill_kernel", "pack_x_kernel", "tile_kernel",
+              "rmsnorm_kernel", "qkv_post_kernel", "attn_partial_kernel", "attn_wide_kernel", "attn_merge_kernel",
+              "add_norm_kernel", "embed_kernel", "head_kernel", "head_fold_kernel", "quant_kernel", "split_x_kernel",
+              "split_fix_kernel", "q4_ffn1_kernel", "ffn1_sum_kernel", "ffn1_vdown_kernel")
 CALIBRATION = "MulFunctor"  # the profile pass's copy: torch.mul(src, 1.0, out=dst)
 
 
@@ -126,8 +126,8 @@ def decode(d: str) -> str:
         n = r["Kernel_Name"]
         us = (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1000.0
         wg = int(r["Grid_Size_X"]) // max(1, int(r["Workgroup_Size_X"]))
-        if "attn_partial" in n:
-            tag = "attention, global" if "512" in n else "attention, sliding"
+        if "attn_partial" in n or "attn_wide" in n:
+            tag = "attention, sliding" if "attn_partial" in n and "512" not in n else "attention, global"
         elif "attn_merge" in n:
             tag = "attention merge"
         elif "head_fold" in n:
